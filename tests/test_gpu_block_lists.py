@@ -1,0 +1,44 @@
+"""The plain walk's 4 x 4 block lists at their edges, on the GPU: every tile
+side with batches of one partial ballot, one, several and more than a thread
+each, over pictures whose last blocks are cut off, and Gaussians the block
+test must not lose -- needles, pixel-sized dots, ones that cover the picture,
+faint ones -- bit for bit against the oracle. The lists are walked two at a
+time, so lists of odd and even length both occur."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from athenea_amd import RenderSettings, TileRasterizer, camera, synthetic
+from tests.test_gpu_parity import check_frame, render_both
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def raster():
+    r = TileRasterizer(0)
+    yield r
+    r.close()
+
+
+def mixed_cloud(n: int, seed: int):
+    """A quarter each: needles, dots, ones that cover the picture, faint ones."""
+    cloud = synthetic.make_cloud(n, seed)
+    kind = np.arange(n) % 4
+    cloud.log_scales[kind == 0] = np.array([-1.0, -6.0, -6.0], np.float32)
+    cloud.log_scales[kind == 1] = -7.0
+    cloud.log_scales[kind == 2] = np.array([0.3, 0.1, -1.0], np.float32)
+    cloud.opacity_logits[kind == 2] = -4.5
+    cloud.opacity_logits[kind == 3] = -5.4  # a little over 1/255
+    return cloud
+
+
+@pytest.mark.parametrize("tile", [8, 16, 32])
+@pytest.mark.parametrize("batch", [32, 96, 256])
+@pytest.mark.parametrize("size", [(101, 67), (3, 130)])
+def test_lists_are_bit_exact(raster, tile, batch, size):
+    print("block lists", tile, batch, size, flush=True)
+    view = camera.view_for(synthetic.front_camera(), *size)
+    settings = RenderSettings(tile=tile, batch=batch)
+    check_frame(*render_both(raster, mixed_cloud(1201, 11), [view], settings, f64=False), f64=False)
