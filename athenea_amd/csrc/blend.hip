@@ -14,9 +14,9 @@
 // front, recovering the transmittance before each Gaussian from the one
 // after it (T_k = T_{k+1} / (1 - alpha_k); alpha <= 0.99 keeps it stable),
 // and accumulates per-slot gradients of the centre, conic, alpha and colour.
-// Lanes of a wavefront walk the same pair at the same step, so a pair's
-// gradient is summed across the wavefront first and added to memory once per
-// wavefront.
+// The 16 lanes of a row walk the same pair at the same step, so a pair's
+// gradient is summed across the row first, then over the tile's rows in LDS,
+// and added to memory once a tile.
 #include "athx_internal.h"
 
 namespace athx {
@@ -160,12 +160,12 @@ __device__ inline uint64_t band_mask(const LdsBatch& s, const Band& B, uint32_t 
     }
 }
 
-// A QUARTER WAVEFRONT'S BLOCK. The plain walk goes finer than the
-// band: each row of 16 lanes owns a 4 x 4 pixel block and walks its own
+// A QUARTER WAVEFRONT'S BLOCK. The plain walk and its adjoint go finer than
+// the band: each row of 16 lanes owns a 4 x 4 pixel block and walks its own
 // list of the staged Gaussians that meet it, so the four rows of a wavefront
 // are at four different Gaussians in the same step, and a wavefront's steps
 // are the longest of its rows' lists instead of the union of what meets 8 x 8
-// pixels. The walk is bound by the VALU's issue rate, so steps are time.
+// pixels. Both kernels are bound by the VALU's issue rate, so steps are time.
 //
 // Which blocks a Gaussian meets is found once, by the thread that staged it:
 // the x-extent of the ellipse q <= C sliced by each row of blocks (the slice
@@ -176,6 +176,11 @@ __device__ inline uint64_t band_mask(const LdsBatch& s, const Band& B, uint32_t 
 // handle meets every block. The answers are one ballot a block and 64
 // Gaussians; each wavefront expands its own blocks' ballots into lists of
 // LDS offsets.
+//
+// A 32 x 32 tile is walked by four workgroups of 16 x 16 pixels (SPLIT 2), each
+// over the tile's pairs for its own quarter: one workgroup of 1024 lanes tests
+// 64 blocks in the few wavefronts that stage, while the others wait (600 k at
+// 1600 x 1100: 403 us a launch, against 8 x 8 pixels a step's 278).
 //
 // Measured against walking what meets a wavefront's 8 x 8 pixels, one Gaussian
 // a step (us a launch, MI355X): 100 k Gaussians at 512 x 512 109 -> 57, 1.4 M
@@ -318,7 +323,7 @@ __device__ inline void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-template <uint32_t TILE, bool kPiped, bool kThreshold>
+template <uint32_t TILE, uint32_t SPLIT, bool kPiped, bool kThreshold>
 __global__ void __launch_bounds__(TILE * TILE) blend_kernel(const DView* __restrict__ views,
                                                             const uint32_t* __restrict__ tile_bases, uint32_t nviews,
                                                             uint32_t batch, const uint32_t* __restrict__ ranges,
@@ -332,19 +337,21 @@ __global__ void __launch_bounds__(TILE * TILE) blend_kernel(const DView* __restr
     // same view at once, so the records gathered at any time are one view's
     // (a working set the 256 MB infinity cache holds, where eight views' do
     // not), and the views' unequal loads even out over the XCDs.
-    const uint32_t gtile = blockIdx.x;
+    const uint32_t gtile = blockIdx.x / (SPLIT * SPLIT), part = blockIdx.x % (SPLIT * SPLIT);
     const uint32_t v = view_of_tile(tile_bases, nviews, gtile);
     const DView& V = views[v];
     const uint32_t local = gtile - V.tile_base;
-    const uint32_t tx = local % V.tiles_x, ty = local / V.tiles_x;
+    // The workgroup's first pixel.
+    const uint32_t ox = ((local % V.tiles_x) * SPLIT + part % SPLIT) * TILE;
+    const uint32_t oy = ((local / V.tiles_x) * SPLIT + part / SPLIT) * TILE;
     const uint32_t tid = threadIdx.x;
     uint32_t lx, ly;
     quarter_pixel<TILE>(tid, lx, ly);
-    const uint32_t px = tx * TILE + lx, py = ty * TILE + ly;
+    const uint32_t px = ox + lx, py = oy + ly;
     const bool inside = px < V.width && py < V.height;
     const uint32_t start = ranges[2 * gtile], end = ranges[2 * gtile + 1];
     const float pxc = (float)px + 0.5f, pyc = (float)py + 0.5f;
-    const float x0 = (float)(tx * TILE) + 0.5f, y0 = (float)(ty * TILE) + 0.5f;
+    const float x0 = (float)ox + 0.5f, y0 = (float)oy + 0.5f;
 
     float r = 0.0f, g = 0.0f, b = 0.0f, T = 1.0f, dsum = 0.0f, dat = -1.0f;
     uint32_t last = 0;
@@ -884,280 +891,275 @@ __global__ void __launch_bounds__(TILE * TILE) contribution_kernel(const DView* 
     }
 }
 
-// The sum over a wavefront's 64 lanes, every lane active: DPP moves within
-// each row of 16 lanes (quad swaps, then rotations by 4 and 8) leave each row's
-// sum in all of its lanes, and four lane reads add the rows. All VALU, no LDS.
-__device__ inline float dpp_add(float x, int ctrl_sel) {
-    int moved = 0;
-    switch (ctrl_sel) {
-    case 0: moved = __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, false); break;   // quad [1,0,3,2]
-    case 1: moved = __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x4E, 0xF, 0xF, false); break;   // quad [2,3,0,1]
-    case 2: moved = __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x124, 0xF, 0xF, false); break;  // row_ror 4
-    default: moved = __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x128, 0xF, 0xF, false); break; // row_ror 8
-    }
-    return x + __builtin_bit_cast(float, moved);
-}
-
-__device__ inline float wave_sum_f(float x) {
-    x = dpp_add(x, 0);
-    x = dpp_add(x, 1);
-    x = dpp_add(x, 2);
-    x = dpp_add(x, 3);
-    const int bits = __builtin_bit_cast(int, x);
-    const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 0));
-    const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 16));
-    const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 32));
-    const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 48));
-    return (r0 + r1) + (r2 + r3);
-}
-
 __device__ inline float as_float(uint32_t u) { return __builtin_bit_cast(float, u); }
 __device__ inline uint32_t as_uint(float f) { return __builtin_bit_cast(uint32_t, f); }
 
-// Eight sums over a wavefront's 64 lanes at once, every lane active (a
-// reduce-scatter): a swap of the wave's halves (v_permlane32_swap) pairs
-// value i with value i + 4 so each lane adds one of them over lanes l and
-// l + 32; a swap of rows within each half (v_permlane16_swap) does the same
-// for the four values left, over l and l + 16; a rotation by 8 within each
-// row of 16, and three DPP steps over each group of 8 lanes, finish. Sum k
-// lands in lane 8k. 26 VALU operations, where eight whole-wave sums take 88.
-__device__ inline float wave_sum8(const float v[8], uint32_t lane) {
-    float r1[4];
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-        const auto p = __builtin_amdgcn_permlane32_swap(as_uint(v[i]), as_uint(v[i + 4]), false, false);
-        r1[i] = as_float(p[0]) + as_float(p[1]);  // lanes 0-31: value i; 32-63: value i + 4
-    }
-    float r2[2];
-#pragma unroll
-    for (uint32_t i = 0; i < 2; ++i) {
-        const auto p = __builtin_amdgcn_permlane16_swap(as_uint(r1[i]), as_uint(r1[i + 2]), false, false);
-        r2[i] = as_float(p[0]) + as_float(p[1]);  // row R of 16 lanes: value i + 2R
-    }
-    const bool upper = (lane & 8u) != 0;
-    const float mine = upper ? r2[1] : r2[0];
-    const float other = upper ? r2[0] : r2[1];
-    float x = mine + as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)as_uint(other), 0x128, 0xF, 0xF, false));
-    x = x + as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)as_uint(x), 0x141, 0xF, 0xF, false));  // half mirror
-    x = dpp_add(x, 1);
-    x = dpp_add(x, 0);
-    return x;
+// Nine sums over each row of 16 lanes at once, the rows apart, every lane of
+// the row active: the DPP adds that halve a value leave the sum in both
+// halves, so where two values are at hand the second's add is written over the
+// first's in half of the row's banks of four lanes (the bank mask), and one
+// register goes on holding both. Bank k of the two registers ends with the
+// sums 2 of its four lanes share: x0 those of v[0], v[2], v[4], v[6] in banks
+// 0 to 3, x1 those of v[1], v[3], v[5], v[7], x2 v[8]'s in every lane: 20 VALU
+// operations for four rows, where whole-wavefront sums of the nine took 39
+// for one Gaussian.
+template <int CTRL>
+__device__ inline float dpp_sum(float x) {
+    return x + as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)as_uint(x), CTRL, 0xF, 0xF, true));
+}
+// dpp_sum(x) in the banks of BANKS, `keep` in the others.
+template <int CTRL, int BANKS>
+__device__ inline float dpp_sum_banks(float x, float keep) {
+    const float sum = x + as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)as_uint(x), CTRL, 0xF, 0xF, true));
+    return as_float((uint32_t)__builtin_amdgcn_update_dpp((int)as_uint(keep), (int)as_uint(sum), 0xE4, 0xF, BANKS, false));
 }
 
-template <uint32_t TILE, bool kPiped>
+__device__ inline void row_sum9(const float (&v)[9], float& x0, float& x1, float& x2) {
+    constexpr int kRor8 = 0x128, kHalfMirror = 0x141, kQuad2301 = 0x4E, kQuad1032 = 0xB1;
+    // Lanes 8-15 (banks 2, 3) go on with v[k + 4].
+    const float a0 = dpp_sum_banks<kRor8, 0xC>(v[4], dpp_sum<kRor8>(v[0]));
+    const float a1 = dpp_sum_banks<kRor8, 0xC>(v[5], dpp_sum<kRor8>(v[1]));
+    const float a2 = dpp_sum_banks<kRor8, 0xC>(v[6], dpp_sum<kRor8>(v[2]));
+    const float a3 = dpp_sum_banks<kRor8, 0xC>(v[7], dpp_sum<kRor8>(v[3]));
+    // Within each half, lanes 4-7 (banks 1, 3) with the value two on.
+    x0 = dpp_sum_banks<kHalfMirror, 0xA>(a2, dpp_sum<kHalfMirror>(a0));
+    x1 = dpp_sum_banks<kHalfMirror, 0xA>(a3, dpp_sum<kHalfMirror>(a1));
+    x0 = dpp_sum<kQuad1032>(dpp_sum<kQuad2301>(x0));
+    x1 = dpp_sum<kQuad1032>(dpp_sum<kQuad2301>(x1));
+    x2 = dpp_sum<kQuad1032>(dpp_sum<kQuad2301>(dpp_sum<kHalfMirror>(dpp_sum<kRor8>(v[8]))));
+}
+
+// Gaussians staged at a time by the adjoint. Every (block, Gaussian) pair of a
+// batch has nine words of LDS for its sums, which no other row writes, since
+// an LDS float add takes some 3 cycles a lane of the CU's LDS pipe (measured:
+// 109 for the 36 lanes of a step, against 7 for a plain write of them; with
+// the adds the walk was bound by that pipe at 95 %): the batch is what leaves
+// room for four workgroups a CU. Measured against the
+// walk of 8 x 8 pixels a step with whole-wavefront sums (us a launch, MI355X):
+// 100 k Gaussians at 512 x 512 293 -> 140, 1.4 M at 1920 x 1080 665 -> 461.
+// Tiles in dispatch order: banded over the XCDs the first takes 183 (the
+// middle bands hold most of the work), the second the same 461.
+template <uint32_t TILE>
+constexpr uint32_t back_batch() {
+    return TILE == 8 ? 32u : 56u;
+}
+
+template <uint32_t TILE, uint32_t SPLIT>
 __global__ void __launch_bounds__(TILE * TILE) blend_backward_kernel(
-    const DView* __restrict__ views, const uint32_t* __restrict__ tile_bases, uint32_t nviews, uint32_t batch,
+    const DView* __restrict__ views, const uint32_t* __restrict__ tile_bases, uint32_t nviews,
     const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ pair_slots, const float* __restrict__ records,
     float* __restrict__ grad2d) {
-    constexpr uint32_t kThreads = TILE * TILE;
-    __shared__ LdsBatch s;
-    __shared__ uint32_t s_slot[kMaxBatch];
-    // The batch's gradients summed over the workgroup's wavefronts, then added
-    // to the slots' words once a batch.
-    __shared__ float s_grad[kMaxBatch * kGrad2d];
+    constexpr uint32_t kThreads = TILE * TILE, kWaves = kThreads / 64;
+    constexpr uint32_t kBx = TILE / 8, kSide = TILE / kBlock, kBlocks = kSide * kSide;
+    constexpr uint32_t batch = back_batch<TILE>();
+    constexpr uint32_t kOut = batch * kGrad2d;  // a block's words
+    static_assert(batch <= 64, "a lane a Gaussian, one ballot");
+    __shared__ LdsWalk<TILE, batch> s;
+    __shared__ uint32_t s_slot[2][64];
+    __shared__ alignas(16) float s_out[kBlocks * kOut];
+    __shared__ float s_sum[kOut];
     __shared__ uint32_t s_max_last;
-    __shared__ uint32_t s_wave_last[kThreads / 64];
-    const uint32_t gtile = xcd_band(blockIdx.x, gridDim.x);
+    const uint32_t gtile = blockIdx.x / (SPLIT * SPLIT), part = blockIdx.x % (SPLIT * SPLIT);
     const uint32_t v = view_of_tile(tile_bases, nviews, gtile);
     const DView& V = views[v];
     const uint32_t local = gtile - V.tile_base;
-    const uint32_t tx = local % V.tiles_x, ty = local / V.tiles_x;
+    const uint32_t ox = ((local % V.tiles_x) * SPLIT + part % SPLIT) * TILE;
+    const uint32_t oy = ((local / V.tiles_x) * SPLIT + part / SPLIT) * TILE;
     const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u;
+    const uint32_t lane = tid & 63u, wave = tid >> 6, row = (tid >> 4) & 3u, q = tid & 15u;
     uint32_t lx, ly;
-    block_pixel<TILE>(tid, lx, ly);
-    const uint32_t px = tx * TILE + lx, py = ty * TILE + ly;
+    quarter_pixel<TILE>(tid, lx, ly);
+    const uint32_t px = ox + lx, py = oy + ly;
     const bool inside = px < V.width && py < V.height;
     const uint32_t start = ranges[2 * gtile];
     const uint32_t tile_pairs = ranges[2 * gtile + 1] - start;
     const float pxc = (float)px + 0.5f, pyc = (float)py + 0.5f;
+    const float x0 = (float)ox + 0.5f, y0 = (float)oy + 0.5f;
     const size_t pix = inside ? (size_t)py * V.width + px : 0;
+    const uint32_t block = ((wave / kBx) * 2u + (row >> 1)) * kSide + (wave % kBx) * 2u + (row & 1u);
 
-    float T = 1.0f, TN = 1.0f;
+    float T = 1.0f;
     uint32_t last = 0;
     float gr = 0.0f, gg = 0.0f, gb = 0.0f, ga = 0.0f;
     if (inside) {
         T = V.final_t[pix];
-        TN = T;
         // A walk never reads past its tile's pairs; the clamp keeps a stale
         // `last` from reading past them either.
         last = min(V.last[pix], tile_pairs);
         const float4 gc = reinterpret_cast<const float4*>(V.dl_dcolour)[pix];
         gr = gc.x; gg = gc.y; gb = gc.z; ga = gc.w;
     }
-    // The colour of everything behind the current Gaussian, as seen from just
-    // in front of it: the background, then each Gaussian over it.
+    // dL/dC . (the colour of everything behind the current Gaussian, as seen
+    // from just in front of it): the background, then each Gaussian over it.
     float br = V.bg[0], bgc = V.bg[1], bb = V.bg[2];
     // d(alpha out)/d(alpha_k) = T_N (1 - bg.a) / (1 - alpha_k).
-    const float ga_scale = ga * TN * (1.0f - V.bg[3]);
+    const float ga_scale = ga * T * (1.0f - V.bg[3]);
     if (tid == 0) {
         s_max_last = 0;
     }
-    if (lane == 0) {
-        s_wave_last[tid >> 6] = 0;
-    }
     __syncthreads();
-    if (last != 0) {
-        atomicMax(&s_max_last, last);
-        atomicMax(&s_wave_last[tid >> 6], last);
+    // A row walks only the pairs below its own pixels' furthest.
+    const uint32_t row_last = row_max(last);
+    if (q == 0 && row_last != 0) {
+        atomicMax(&s_max_last, row_last);
     }
     __syncthreads();
     const uint32_t max_last = s_max_last;
-    // A wavefront walks only the pairs below its own pixels' furthest.
-    const uint32_t wave_last = s_wave_last[tid >> 6];
-    const Band band = wave_band<TILE>(V, tx, ty, tid >> 6);
-    // kPiped: the staging runs a batch ahead of the walk, as in the forward
-    // blend -- while a batch is walked each thread reads its record of the
-    // next (lower) batch and its slot of the one after. The reads are
-    // unconditional, at in-bounds pairs of the tile (the tile has max_last
-    // pairs or more).
+    // The lanes that write a row's sums: lanes 0 and 1 of each bank x0's and
+    // x1's, lane 2 of the first x2's; their words within a Gaussian's: u, u dx,
+    // u dx dx, u dx dy, u dy, u dy dy, then w dL/d(r, g, b).
+    const bool writes = (q & 3u) < 2u || q == 2u;
+    float* const out = s_out + block * kOut + (q == 2u ? 8u : (q >> 2) * 2u + (q & 1u));
+    // The staging runs a batch ahead of the walk, as in the forward blend:
+    // while a batch is walked each lane reads its record of the next (lower)
+    // batch and its slot of the one after. Every wavefront reads them all, since
+    // each tests rows of blocks of its own. The reads are unconditional, at
+    // in-bounds pairs of the tile (the tile has max_last pairs or more).
     const auto pair_of = [&](uint32_t hi_b) {
         const uint32_t lo_b = hi_b > batch ? hi_b - batch : 0u;
-        const uint32_t k = lo_b + tid;
+        const uint32_t k = lo_b + lane;
         return start + (k < hi_b ? k : (hi_b != 0u ? hi_b - 1u : 0u));
     };
     uint32_t slot_now = 0, slot_ahead = 0;
     Staged rec_now{};
-    if (kPiped && max_last > 0) {
+    if (max_last > 0) {
         slot_now = pair_slots[pair_of(max_last)];
         rec_now = fetch(records, slot_now);
-        const uint32_t hi1 = max_last > batch ? max_last - batch : 0u;
-        slot_ahead = pair_slots[pair_of(hi1)];
+        slot_ahead = pair_slots[pair_of(max_last > batch ? max_last - batch : 0u)];
     }
-    for (uint32_t hi = max_last; hi > 0;) {
+    const auto clear_out = [&]() {
+        for (uint32_t k = tid; k < kBlocks * kOut / 4u; k += kThreads) {
+            reinterpret_cast<float4*>(s_out)[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+    };
+    static_assert(kBlocks * kOut % 4u == 0, "cleared by 16-byte words");
+    clear_out();
+    uint32_t turn = 0;
+    for (uint32_t hi = max_last; hi > 0; turn ^= 1u) {
         const uint32_t lo = hi > batch ? hi - batch : 0;
         const uint32_t count = hi - lo;
-        if constexpr (kPiped) {
-            if (tid < count) {
-                s_slot[tid] = slot_now;
-                put(s, tid, rec_now);
-            }
-        } else {
-            for (uint32_t k = tid; k < count; k += kThreads) {
-                const uint32_t slot = pair_slots[start + lo + k];
-                s_slot[k] = slot;
-                stage(s, k, records, slot);
-            }
+        if (wave == 0 && lane < count) {
+            s_slot[turn][lane] = slot_now;
+            put(s.rec[lane], rec_now);
         }
-        for (uint32_t k = tid; k < count * kGrad2d; k += kThreads) {
-            s_grad[k] = 0.0f;
+        for (uint32_t slice = wave; slice < kSide; slice += kWaves) {
+            blocks_met<TILE, 1>(rec_now, lane < count, x0, y0, lane, s.meets[0], slice);
         }
         __syncthreads();
-        if constexpr (kPiped) {
-            // The next batch is [lo - batch, lo); the one after it ends where
-            // that one starts.
-            slot_now = slot_ahead;
-            rec_now = fetch(records, slot_ahead);
-            const uint32_t lo1 = lo > batch ? lo - batch : 0u;
-            slot_ahead = pair_slots[pair_of(lo1)];
+        // The next batch is [lo - batch, lo); the one after it ends where that
+        // one starts.
+        slot_now = slot_ahead;
+        rec_now = fetch(records, slot_ahead);
+        slot_ahead = pair_slots[pair_of(lo > batch ? lo - batch : 0u)];
+        // Back to front over the row's Gaussians below its furthest pair.
+        const uint32_t top = row_last > lo ? (row_last - lo < count ? row_last - lo : count) : 0u;
+        const uint32_t length = expand_list(s, block, lane, top);
+        wave_lds_fence();
+        const uint16_t* list = s.list[block];
+        const uint32_t last_at = last > lo ? (last - lo) * (uint32_t)sizeof(LdsRecord) : 0u;
+        for (uint32_t i = length; i-- != 0;) {
+            const uint32_t at = list[i];
+            const LdsRecord& k = *reinterpret_cast<const LdsRecord*>(reinterpret_cast<const char*>(s.rec) + at);
+            const float4 ka = k.a, kb = k.b, kc = k.c;
+            const float dx = pxc - ka.x, dy = pyc - ka.y;
+            const float x = ka.z * dx * dx + ka.w * dx * dy + kb.x * dy * dy;
+            const float e = blend_exp_of(x);
+            const float raw = kb.z * e;
+            const float clamped = fminf(0.99f, raw);
+            const bool took = (at < last_at) & !(x < kb.y) & !(clamped < 1.0f / 255.0f);
+            // A lane that did not take the Gaussian goes through with an alpha
+            // of 0 (T and the colour behind it unchanged, every term 0).
+            const float alpha = took ? clamped : 0.0f;
+            const float one_minus = 1.0f - alpha;
+            // 1 / (1 - alpha), alpha <= 0.99: the hardware reciprocal and one
+            // Newton step (within an ulp or so of the quotient), where an IEEE
+            // divide takes a dozen operations. The adjoint answers to finite
+            // differences at 1e-3, not to bits.
+            float inv = __builtin_amdgcn_rcpf(one_minus);
+            inv = __builtin_fmaf(inv, __builtin_fmaf(-one_minus, inv, 1.0f), inv);
+            T = T * inv;
+            const float or_ = took ? kc.x - br : 0.0f, og = took ? kc.y - bgc : 0.0f, ob = took ? kc.z - bb : 0.0f;
+            const float over = __builtin_fmaf(or_, gr, __builtin_fmaf(og, gg, ob * gb));
+            const float dl_dalpha = __builtin_fmaf(T, over, ga_scale * inv);
+            br = __builtin_fmaf(alpha, or_, br);
+            bgc = __builtin_fmaf(alpha, og, bgc);
+            bb = __builtin_fmaf(alpha, ob, bb);
+            const float w = alpha * T;
+            const float u = dl_dalpha * (took & !(raw > 0.99f) ? e : 0.0f);
+            const float ux = u * dx, uy = u * dy;
+            // -2 x's derivatives along dx and dy, where a thin Gaussian's
+            // terms cancel: taken a pixel, not from the pixels' sums.
+            const float hx = __builtin_fmaf(-ka.w, dy, -2.0f * (ka.z * dx));
+            const float hy = __builtin_fmaf(-ka.w, dx, -2.0f * (kb.x * dy));
+            const float sums[9] = {u, u * hx, ux * dx, ux * dy, u * hy, uy * dy, w * gr, w * gg, w * gb};
+            float s0, s1, s2;
+            row_sum9(sums, s0, s1, s2);
+            if (writes) {
+                // (at is 48 bytes a Gaussian, its words 36.)
+                static_assert(sizeof(LdsRecord) * 3 == kGrad2d * sizeof(float) * 4, "48 to 36");
+                *reinterpret_cast<float*>(reinterpret_cast<char*>(out) + (at - (at >> 2))) =
+                    q == 2u ? s2 : (q & 1u) ? s1 : s0;
+            }
         }
-        const uint32_t top = wave_last > lo ? (wave_last - lo < count ? wave_last - lo : count) : 0u;
-        // Back to front over the pairs below `top` that meet the band, 64 at a
-        // time; the rest hold no pixel of it and add nothing.
-        for (uint32_t c1 = top; c1 > 0; c1 = c1 > 64u ? c1 - 64u : 0u) {
-          const uint32_t c0 = c1 > 64u ? c1 - 64u : 0u;
-          for (uint64_t mm = band_mask<TILE>(s, band, c0, c1, lane); mm != 0;) {
-            const uint32_t bit = 63u - (uint32_t)__builtin_clzll(mm);
-            mm &= ~(1ull << bit);
-            const uint32_t j = c0 + bit;
-            const uint32_t idx = lo + j;
-            bool contrib = false;
-            float g_cx = 0.f, g_cy = 0.f, g_ka = 0.f, g_kb = 0.f, g_kc = 0.f, g_al = 0.f, g_r = 0.f, g_g = 0.f,
-                  g_b = 0.f;
-            if (idx < last) {
-                const float4 q = s.xy_cut_op[j];
-                const float4 k = s.conic[j];
-                const float dx = pxc - q.x, dy = pyc - q.y;
-                const float power = k.x * dx * dx + k.y * dx * dy + k.z * dy * dy;
-                if (power <= q.z) {
-                    const float e = blend_exp(power);
-                    const float raw = q.w * e;
-                    const float alpha = fminf(0.99f, raw);
-                    if (alpha >= 1.0f / 255.0f) {
-                        contrib = true;
-                        const float4 c = s.colour[j];
-                        const float one_minus = 1.0f - alpha;
-                        // 1 / (1 - alpha), alpha <= 0.99: the hardware
-                        // reciprocal and one Newton step (within an ulp or so
-                        // of the quotient), where an IEEE divide takes a dozen
-                        // operations twice a pair. The adjoint answers to
-                        // finite differences at 1e-3, not to bits.
-                        float inv = __builtin_amdgcn_rcpf(one_minus);
-                        inv = inv + inv * (1.0f - one_minus * inv);
-                        const float Tb = T * inv;
-                        const float w = alpha * Tb;
-                        g_r = w * gr;
-                        g_g = w * gg;
-                        g_b = w * gb;
-                        const float dl_dalpha =
-                            Tb * ((c.x - br) * gr + (c.y - bgc) * gg + (c.z - bb) * gb) + ga_scale * inv;
-                        br = c.x * alpha + br * one_minus;
-                        bgc = c.y * alpha + bgc * one_minus;
-                        bb = c.z * alpha + bb * one_minus;
-                        T = Tb;
-                        if (!(raw > 0.99f)) {
-                            g_al = dl_dalpha * e;
-                            const float dl_dpower = dl_dalpha * (-0.5f * alpha);
-                            const float kb = c.w;
-                            g_ka = dl_dpower * dx * dx;
-                            g_kb = dl_dpower * 2.0f * dx * dy;
-                            g_kc = dl_dpower * dy * dy;
-                            // power depends on the centre through dx = px - cx.
-                            g_cx = -dl_dpower * (2.0f * k.x * dx + 2.0f * kb * dy);
-                            g_cy = -dl_dpower * (2.0f * kb * dx + 2.0f * k.z * dy);
-                        }
-                    }
-                }
+        __syncthreads();
+        // Each Gaussian's words summed over the tile's blocks.
+        for (uint32_t k = tid; k < count * kGrad2d; k += kThreads) {
+            float sum = 0.0f;
+#pragma unroll 8
+            for (uint32_t m = 0; m < kBlocks; ++m) {
+                sum += s_out[m * kOut + k];
             }
-            if (__any(contrib)) {
-                const float eight[8] = {g_cx, g_cy, g_ka, g_kb, g_kc, g_al, g_r, g_g};
-                const float sum8 = wave_sum8(eight, lane);
-                const float sum_b = wave_sum_f(g_b);
-                if ((lane & 7u) == 0) {
-                    atomicAdd(&s_grad[j * kGrad2d + (lane >> 3)], sum8);
-                } else if (lane == 1) {
-                    atomicAdd(&s_grad[j * kGrad2d + 8], sum_b);
-                }
-            }
-          }
+            s_sum[k] = sum;
+        }
+        __syncthreads();
+        clear_out();
+        // The exponent x = -(a dx dx + 2 b dx dy + c dy dy) / 2 taken apart, in
+        // place: to the centre, conic and alpha (kGrad2d's order).
+        for (uint32_t k = tid; k < count; k += kThreads) {
+            float* G = s_sum + k * kGrad2d;
+            const LdsRecord& p = s.rec[k];
+            const float op = p.b.z;
+            const float u = G[0], ux = G[1], uxx = G[2], uxy = G[3], uy = G[4], uyy = G[5];
+            G[0] = op * ux;
+            G[1] = op * uy;
+            G[2] = -0.5f * op * uxx;
+            G[3] = -op * uxy;
+            G[4] = -0.5f * op * uyy;
+            G[5] = u;
         }
         __syncthreads();
         for (uint32_t k = tid; k < count * kGrad2d; k += kThreads) {
-            const float g = s_grad[k];
+            const uint32_t j = k / kGrad2d;
+            const float g = s_sum[k];
             if (g != 0.0f) {
-                atomicAdd(&grad2d[(size_t)s_slot[k / kGrad2d] * kGrad2d + k % kGrad2d], g);
+                atomicAdd(&grad2d[(size_t)s_slot[turn][j] * kGrad2d + (k - j * kGrad2d)], g);
             }
         }
-        __syncthreads();
         hi = lo;
     }
 }
 
-template <uint32_t TILE>
+template <uint32_t TILE, uint32_t SPLIT>
 hipError_t blend_for(const DView* views, const uint32_t* tile_bases, uint32_t nviews, uint32_t tiles, uint32_t batch,
                      const uint32_t* ranges, const uint32_t* slots, const float* records, uint32_t depth_mode,
                      float depth_threshold, hipStream_t s) {
     using Kernel = void (*)(const DView*, const uint32_t*, uint32_t, uint32_t, const uint32_t*, const uint32_t*,
                             const float*, uint32_t, float);
     const bool piped = batch <= TILE * TILE, threshold = depth_mode != 0;
-    const Kernel kernel = piped ? (threshold ? blend_kernel<TILE, true, true> : blend_kernel<TILE, true, false>)
-                                : (threshold ? blend_kernel<TILE, false, true> : blend_kernel<TILE, false, false>);
-    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(TILE * TILE), 0, s, views, tile_bases, nviews, batch, ranges, slots,
-                       records, depth_mode, depth_threshold);
+    const Kernel kernel =
+        piped ? (threshold ? blend_kernel<TILE, SPLIT, true, true> : blend_kernel<TILE, SPLIT, true, false>)
+              : (threshold ? blend_kernel<TILE, SPLIT, false, true> : blend_kernel<TILE, SPLIT, false, false>);
+    hipLaunchKernelGGL(kernel, dim3(tiles * SPLIT * SPLIT), dim3(TILE * TILE), 0, s, views, tile_bases, nviews, batch,
+                       ranges, slots, records, depth_mode, depth_threshold);
     return hipGetLastError();
 }
 
-template <uint32_t TILE>
+template <uint32_t TILE, uint32_t SPLIT>
 hipError_t blend_backward_for(const DView* views, const uint32_t* tile_bases, uint32_t nviews, uint32_t tiles,
-                              uint32_t batch, const uint32_t* ranges, const uint32_t* slots, const float* records,
-                              float* grad2d, hipStream_t s) {
-    if (batch <= TILE * TILE) {
-        hipLaunchKernelGGL((blend_backward_kernel<TILE, true>), dim3(tiles), dim3(TILE * TILE), 0, s, views,
-                           tile_bases, nviews, batch, ranges, slots, records, grad2d);
-    } else {
-        hipLaunchKernelGGL((blend_backward_kernel<TILE, false>), dim3(tiles), dim3(TILE * TILE), 0, s, views,
-                           tile_bases, nviews, batch, ranges, slots, records, grad2d);
-    }
+                              const uint32_t* ranges, const uint32_t* slots, const float* records, float* grad2d,
+                              hipStream_t s) {
+    hipLaunchKernelGGL((blend_backward_kernel<TILE, SPLIT>), dim3(tiles * SPLIT * SPLIT), dim3(TILE * TILE), 0, s,
+                       views, tile_bases, nviews, ranges, slots, records, grad2d);
     return hipGetLastError();
 }
 
@@ -1187,13 +1189,13 @@ hipError_t launch_blend(const DView* views_dev, const uint32_t* tile_bases, uint
     }
     switch (tile) {
     case 8:
-        return blend_for<8>(views_dev, tile_bases, nviews, total_tiles, batch, ranges, pair_slots, records, depth_mode,
+        return blend_for<8, 1>(views_dev, tile_bases, nviews, total_tiles, batch, ranges, pair_slots, records, depth_mode,
                             depth_threshold, s);
     case 16:
-        return blend_for<16>(views_dev, tile_bases, nviews, total_tiles, batch, ranges, pair_slots, records,
+        return blend_for<16, 1>(views_dev, tile_bases, nviews, total_tiles, batch, ranges, pair_slots, records,
                              depth_mode, depth_threshold, s);
     case 32:
-        return blend_for<32>(views_dev, tile_bases, nviews, total_tiles, batch, ranges, pair_slots, records,
+        return blend_for<16, 2>(views_dev, tile_bases, nviews, total_tiles, batch, ranges, pair_slots, records,
                              depth_mode, depth_threshold, s);
     default:
         return hipErrorInvalidValue;
@@ -1256,13 +1258,13 @@ hipError_t launch_blend_backward(const DView* views_dev, const uint32_t* tile_ba
     }
     switch (tile) {
     case 8:
-        return blend_backward_for<8>(views_dev, tile_bases, nviews, total_tiles, batch, ranges, pair_slots, records,
+        return blend_backward_for<8, 1>(views_dev, tile_bases, nviews, total_tiles, ranges, pair_slots, records,
                                      grad2d, s);
     case 16:
-        return blend_backward_for<16>(views_dev, tile_bases, nviews, total_tiles, batch, ranges, pair_slots, records,
+        return blend_backward_for<16, 1>(views_dev, tile_bases, nviews, total_tiles, ranges, pair_slots, records,
                                       grad2d, s);
     case 32:
-        return blend_backward_for<32>(views_dev, tile_bases, nviews, total_tiles, batch, ranges, pair_slots, records,
+        return blend_backward_for<16, 2>(views_dev, tile_bases, nviews, total_tiles, ranges, pair_slots, records,
                                       grad2d, s);
     default:
         return hipErrorInvalidValue;

@@ -3,13 +3,15 @@ side with batches of one partial ballot, one, several and more than a thread
 each, over pictures whose last blocks are cut off, and Gaussians the block
 test must not lose -- needles, pixel-sized dots, ones that cover the picture,
 faint ones -- bit for bit against the oracle. The lists are walked two at a
-time, so lists of odd and even length both occur."""
+time, so lists of odd and even length both occur. The adjoint's batches below."""
 from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 from athenea_amd import RenderSettings, TileRasterizer, camera, synthetic
+from athenea_amd.autograd import rasterize
 from tests.test_gpu_parity import check_frame, render_both
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +44,28 @@ def test_lists_are_bit_exact(raster, tile, batch, size):
     view = camera.view_for(synthetic.front_camera(), *size)
     settings = RenderSettings(tile=tile, batch=batch)
     check_frame(*render_both(raster, mixed_cloud(1201, 11), [view], settings, f64=False), f64=False)
+
+
+def gradients(raster, cloud, view, dl, settings):
+    params = [torch.from_numpy(a).cuda().requires_grad_(True) for a in
+              (cloud.means, cloud.log_scales, cloud.quats, cloud.opacity_logits, cloud.sh)]
+    colours, _ = rasterize(*params, [view], raster, settings)
+    return [g.double() for g in torch.autograd.grad(colours, params, [dl])]
+
+
+@pytest.mark.parametrize("size", [(101, 67), (3, 130)])
+def test_adjoint_over_several_batches(raster, size):
+    """Tiles of hundreds of pairs, many batches of every tile side's adjoint
+    (32, 56 and 24 Gaussians): the gradients of one picture do not depend on
+    how its pairs are cut up. Each is a sum of at most a few thousand float
+    products in another order, so they agree to a few thousand units of 2^-24
+    of the largest."""
+    print("adjoint batches", size, flush=True)
+    view = camera.view_for(synthetic.front_camera(), *size)
+    cloud = mixed_cloud(3001, 12)
+    dl = torch.randn((size[1], size[0], 4), generator=torch.Generator(device="cuda").manual_seed(3), device="cuda")
+    base = gradients(raster, cloud, view, dl, RenderSettings(tile=16))
+    for tile in (8, 32):
+        for got, want in zip(gradients(raster, cloud, view, dl, RenderSettings(tile=tile)), base):
+            assert torch.isfinite(got).all()
+            assert float((got - want).norm()) <= 4096 * 2.0**-24 * float(want.norm())
