@@ -23,12 +23,12 @@ namespace {
 constexpr uint32_t kThreads = 256;
 constexpr uint32_t kWaves = kThreads / 64;
 constexpr uint32_t kItems = 16;
-constexpr uint32_t kPart = kThreads * kItems;
 constexpr uint32_t kRadix = 256;
 constexpr uint32_t kMaxPasses = 8;
 constexpr uint32_t kFlagAggregate = 1u << 30;
 constexpr uint32_t kFlagPrefix = 2u << 30;
 constexpr uint32_t kValueMask = (1u << 30) - 1;
+constexpr uint32_t kLook = 8;  // predecessors a look-back step reads
 
 __device__ inline uint32_t load_word(const uint32_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -63,6 +63,18 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t x, uint32_t* s_tmp, uin
     __syncthreads();
     total = all;
     return before + incl - x;
+}
+
+// The onesweep partition a sort of `cap` keys takes: 1024 keys up to
+// kSmallSort, 4096 beyond. A few thousand to a few hundred thousand keys are
+// few partitions of 4096, each a CU's whole latency chain (ranking 16 keys a
+// lane one after another) on a tenth of the chip: four times the partitions
+// take a quarter of the chain. Measured, us a pass of 4 k and 100 k keys:
+// 11.0 and 14.2 with 4096 and one predecessor a look-back step, 5.9 and 9.9
+// with 1024 and kLook; 1.3 M keys take 24.4 and (4096, kLook) 22.8.
+constexpr uint32_t kSmallSort = 1u << 19;
+__host__ __device__ inline uint32_t onesweep_part(uint32_t cap) {
+    return cap <= kSmallSort ? kThreads * 4u : kThreads * kItems;
 }
 
 // The pair count lives in device memory (the scan's total), bounded by the
@@ -169,7 +181,7 @@ __global__ void __launch_bounds__(kThreads) hist_reduce_kernel(const uint32_t* _
     }
 }
 
-template <typename K>
+template <typename K, uint32_t ITEMS>
 __global__ void __launch_bounds__(kThreads) onesweep_kernel(const K* __restrict__ kin,
                                                             const uint32_t* __restrict__ vin,
                                                             K* __restrict__ kout, uint32_t* __restrict__ vout,
@@ -178,6 +190,7 @@ __global__ void __launch_bounds__(kThreads) onesweep_kernel(const K* __restrict_
                                                             const uint32_t* __restrict__ hist,
                                                             uint32_t* __restrict__ lookback,
                                                             uint32_t* __restrict__ counter) {
+    constexpr uint32_t kPart = kThreads * ITEMS;
     __shared__ K s_keys[kPart];
     __shared__ uint32_t s_vals[kPart];
     __shared__ uint32_t s_wave_hist[kWaves * kRadix];
@@ -205,15 +218,15 @@ __global__ void __launch_bounds__(kThreads) onesweep_kernel(const K* __restrict_
         return;
     }
     const uint32_t part_first = part * kPart;
-    const uint32_t wave_first = part_first + wave * (64 * kItems);
+    const uint32_t wave_first = part_first + wave * (64 * ITEMS);
 
     // Load: item j of a lane sits at wave_first + j * 64 + lane, so the order
     // of the input is (wave, j, lane) and ranking j by j keeps it stable.
-    K key[kItems];
-    uint32_t val[kItems];
-    uint32_t rank[kItems];
+    K key[ITEMS];
+    uint32_t val[ITEMS];
+    uint32_t rank[ITEMS];
 #pragma unroll
-    for (uint32_t j = 0; j < kItems; ++j) {
+    for (uint32_t j = 0; j < ITEMS; ++j) {
         const uint32_t at = wave_first + j * 64 + lane;
         const bool ok = at < n;
         key[j] = ok ? kin[at] : 0;
@@ -223,7 +236,7 @@ __global__ void __launch_bounds__(kThreads) onesweep_kernel(const K* __restrict_
     const uint32_t dmask = (1u << width) - 1u;
     uint32_t* my_hist = s_wave_hist + wave * kRadix;
 #pragma unroll
-    for (uint32_t j = 0; j < kItems; ++j) {
+    for (uint32_t j = 0; j < ITEMS; ++j) {
         const uint32_t at = wave_first + j * 64 + lane;
         const bool ok = at < n;
         const uint32_t d = (uint32_t)(key[j] >> shift) & dmask;
@@ -260,19 +273,30 @@ __global__ void __launch_bounds__(kThreads) onesweep_kernel(const K* __restrict_
     const uint32_t global_start = block_exclusive_scan(hist[d], s_tmp, unused);
     uint32_t before = 0;
     if (part != 0 && digit) {
-        int32_t j = (int32_t)part - 1;
-        while (true) {
-            uint32_t w = load_word(lookback + (size_t)j * kRadix + d);
-            // Partition j took its ticket before this one: it publishes.
-            while ((w >> 30) == 0) {
-                __builtin_amdgcn_s_sleep(1);
-                w = load_word(lookback + (size_t)j * kRadix + d);
+        // kLook predecessors' words a step, read together: one at a time, a
+        // frame's few partitions (all in flight at once) waited out half their
+        // number of memory latencies.
+        bool found = false;
+        for (int32_t j = (int32_t)part - 1; !found; j -= (int32_t)kLook) {
+            uint32_t w[kLook];
+#pragma unroll
+            for (uint32_t u = 0; u < kLook; ++u) {
+                const int32_t at = j - (int32_t)u;
+                w[u] = load_word(lookback + (size_t)(at > 0 ? at : 0) * kRadix + d);
             }
-            before += w & kValueMask;
-            if ((w >> 30) == 2u || j == 0) {
-                break;
+#pragma unroll
+            for (uint32_t u = 0; u < kLook; ++u) {
+                const int32_t at = j - (int32_t)u;
+                if (!found) {
+                    // Partition `at` took its ticket before this one: it publishes.
+                    while ((w[u] >> 30) == 0) {
+                        __builtin_amdgcn_s_sleep(1);
+                        w[u] = load_word(lookback + (size_t)at * kRadix + d);
+                    }
+                    before += w[u] & kValueMask;
+                    found = (w[u] >> 30) == 2u || at == 0;
+                }
             }
-            --j;
         }
         store_word(my_word, kFlagPrefix | ((before + count) & kValueMask));
     }
@@ -282,7 +306,7 @@ __global__ void __launch_bounds__(kThreads) onesweep_kernel(const K* __restrict_
     // Into LDS in digit order, then out: each digit's run is contiguous in
     // the output, so neighbouring threads write neighbouring addresses.
 #pragma unroll
-    for (uint32_t j = 0; j < kItems; ++j) {
+    for (uint32_t j = 0; j < ITEMS; ++j) {
         const uint32_t at = wave_first + j * 64 + lane;
         if (at < n) {
             const uint32_t dj = (uint32_t)(key[j] >> shift) & dmask;
@@ -556,8 +580,9 @@ __global__ void __launch_bounds__(kT) downsweep_kernel(const K* __restrict__ kin
 __global__ void clear_kernel(uint32_t* __restrict__ lookback, uint32_t* __restrict__ counters, uint32_t passes,
                              const uint64_t* __restrict__ n_dev, uint32_t cap) {
     const uint32_t n = count_of(n_dev, cap);
-    const uint64_t parts_cap = div_up(cap ? cap : 1, kPart);
-    const uint64_t per_pass = (uint64_t)div_up(n ? n : 1, kPart) * kRadix;
+    const uint32_t part = onesweep_part(cap);
+    const uint64_t parts_cap = div_up(cap ? cap : 1, part);
+    const uint64_t per_pass = (uint64_t)div_up(n ? n : 1, part) * kRadix;
     const uint64_t look = (uint64_t)passes * per_pass;
     const uint64_t total = look + passes;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (uint64_t)gridDim.x * blockDim.x) {
@@ -652,9 +677,9 @@ hipError_t sort_impl(K* keys, uint32_t* values, const uint64_t* n_dev, uint32_t 
     for (uint32_t p = 0; p < passes; ++p) {
         uint32_t shift, width;
         pass_digit(p, lo_bit, key_bits - lo_bit, passes, shift, width);
-        hipLaunchKernelGGL(onesweep_kernel<K>, dim3(parts), dim3(kThreads), 0, s, kin, vin, kout, vout, n_dev, cap,
-                           shift, width, sc.hist + p * kRadix, sc.lookback + (size_t)p * parts * kRadix,
-                           sc.counters + p);
+        hipLaunchKernelGGL((cap <= kSmallSort ? onesweep_kernel<K, 4> : onesweep_kernel<K, kItems>), dim3(parts),
+                           dim3(kThreads), 0, s, kin, vin, kout, vout, n_dev, cap, shift, width, sc.hist + p * kRadix,
+                           sc.lookback + (size_t)p * parts * kRadix, sc.counters + p);
         K* tk = kin; kin = kout; kout = tk;
         uint32_t* tv = vin; vin = vout; vout = tv;
     }
@@ -670,7 +695,7 @@ hipError_t sort_impl(K* keys, uint32_t* values, const uint64_t* n_dev, uint32_t 
 
 }  // namespace
 
-uint32_t sort_partitions(uint32_t n) { return div_up(n ? n : 1, kPart); }
+uint32_t sort_partitions(uint32_t n) { return div_up(n ? n : 1, onesweep_part(n)); }
 
 uint32_t sort_hist_blocks(uint32_t n) {
     const uint32_t parts = sort_partitions(n);
