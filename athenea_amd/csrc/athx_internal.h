@@ -256,7 +256,8 @@ struct StripBins {
 hipError_t launch_strip_mask_emit(const DView* views_dev, uint32_t n, uint32_t tile, const uint32_t* sorted_slots,
                                   const uint32_t* offsets, const uint64_t* visible_dev, uint32_t max_visible,
                                   uint32_t cap, const float* records, uint32_t* strip_keys, uint32_t* strip_slots,
-                                  uint32_t* rank_tiles, hipStream_t s, uint32_t* view_entry = nullptr);
+                                  uint32_t* rank_tiles, hipStream_t s, uint32_t* view_entry = nullptr,
+                                  uint64_t* tally = nullptr);
 // Each strip's segments, scanned: segbase[s] and the total in *seg_total.
 hipError_t launch_seg_scan(const uint32_t* strip_ranges, uint32_t strips, uint32_t* segbase, uint64_t* seg_total,
                            uint32_t* status_words, hipStream_t s);
@@ -285,7 +286,8 @@ hipError_t launch_scan(const uint32_t* in, uint32_t* out, uint64_t* total, uint3
 // [start, end) of every key in 0..keys-1 among the first min(*n_dev, cap)
 // sorted keys (compared under key_mask); (0, 0) for a key that is absent.
 hipError_t launch_ranges(const uint32_t* sorted_keys, const uint64_t* n_dev, uint32_t cap, uint32_t keys,
-                         uint32_t* ranges, hipStream_t s, uint32_t key_mask = ~0u);
+                         uint32_t* ranges, hipStream_t s, uint32_t key_mask = ~0u, const uint64_t* tally = nullptr,
+                         uint64_t* pair_total = nullptr);
 // The reference's 64-bit pair keys of the tile-sorted pairs: tile << 24 |
 // the depth key of the pair's slot, a workgroup a tile over its range.
 hipError_t launch_pair_keys(const uint32_t* ranges, uint32_t tiles, const uint32_t* values,
@@ -294,6 +296,47 @@ hipError_t launch_blend(const DView* views_dev, const uint32_t* view_of_tile_bas
                         uint32_t total_tiles, uint32_t tile, uint32_t batch, const uint32_t* ranges,
                         const uint32_t* pair_slots, const float* records, uint32_t depth_mode, float depth_threshold,
                         hipStream_t s, bool variants = false, const uint32_t* slot_ids = nullptr);
+// The sorted strip entries as a walk reads them: each strip's range, each
+// entry's tile mask (the keys' upper halves where masks is null) and slot.
+struct EntryWalk {
+    const uint32_t* ranges;
+    const uint32_t* keys;
+    const uint16_t* masks;
+    const uint32_t* slots;
+};
+// The plain blend from the entries themselves, no pairs listed (tiles of 16
+// or 32 pixels).
+hipError_t launch_blend_entries(const DView* views_dev, const uint32_t* tile_bases, uint32_t nviews,
+                                uint32_t total_tiles, uint32_t tile, const EntryWalk& entries, const float* records,
+                                uint32_t depth_mode, float depth_threshold, hipStream_t s);
+// The pairs of a frame that lists none: each wavefront of the emission adds its
+// entries' mask bits to one of kTallyWords words, kTallyStride apart (an atomic
+// on one address takes some 11.5 ns: one word a frame would serialise them),
+// which the settle pass clears before it and the strip ranges' kernel adds up
+// after it.
+constexpr uint32_t kTallyWords = 1024, kTallyStride = 8;
+// Their sum to *pair_total, by a kernel's first workgroup (of 256 lanes, all
+// of them here).
+__device__ inline void sum_tally(const uint64_t* tally, uint64_t* pair_total) {
+    __shared__ uint64_t s_tally[4];
+    if (!tally || blockIdx.x != 0) {
+        return;
+    }
+    uint64_t x = 0;
+    for (uint32_t w = threadIdx.x; w < kTallyWords; w += 256u) {
+        x += tally[w * kTallyStride];
+    }
+    for (uint32_t d = 32; d >= 1; d >>= 1) {
+        x += __shfl_xor(x, d, 64);
+    }
+    if ((threadIdx.x & 63u) == 0) {
+        s_tally[threadIdx.x >> 6] = x;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        *pair_total = s_tally[0] + s_tally[1] + s_tally[2] + s_tally[3];
+    }
+}
 // What each splat gave the last frame's walk (the frame's ranges, pair
 // slots and records): mode 1 the blend weight in 1/4096, one word a slot;
 // mode 4 the colour gradient against each view's dl_dcolour in 1/256 (three
@@ -385,7 +428,8 @@ hipError_t launch_segment_sort(uint32_t* keys, uint32_t* values, const SegmentAr
 // empty) from its scanned counts (radix digits a partition).
 hipError_t launch_strip_ranges_seg(const uint32_t* offsets, const SegmentArgs& g, uint32_t nviews,
                                    const uint32_t* strip_bases, uint32_t strips, uint32_t radix,
-                                   const uint64_t* total_dev, uint32_t* ranges, hipStream_t s);
+                                   const uint64_t* total_dev, uint32_t* ranges, hipStream_t s,
+                                   const uint64_t* tally = nullptr, uint64_t* pair_total = nullptr);
 constexpr uint32_t kMaxSegmentViews = 256;
 struct SegmentBuild {
     uint32_t nviews;
@@ -414,7 +458,8 @@ constexpr uint32_t kCompactTile = 4096;
 // The unsettled footprints settled (launch_project leaves them), and each
 // block's drawn slots counted into sums (the compaction's status words).
 hipError_t launch_settle_count(const DView* views_dev, uint32_t n, uint32_t tile, uint32_t slots, const float* records,
-                               uint32_t* touched, uint32_t* depth_keys, uint64_t* sums, hipStream_t s);
+                               uint32_t* touched, uint32_t* depth_keys, uint64_t* sums, hipStream_t s,
+                               uint64_t* tally = nullptr);
 // The visible slots in slot order with their depth keys (each key's top byte
 // holding the slot's strip-entry count, capped at 255); the count lands in
 // *visible_total (device). counted: the blocks' counts are already in the

@@ -74,6 +74,38 @@ uint32_t bits_for(uint32_t values) {
     return bits;
 }
 
+// The sizes a frame runs at.
+struct FrameShape {
+    uint32_t nviews = 0;
+    uint32_t instances = 1;    // clouds projected into each view
+    uint32_t count = 0;        // Gaussians a view: every instance's, back to back
+    uint32_t slots = 0;        // views * count
+    uint32_t tiles = 0;        // over all views
+    uint32_t strips = 0;       // over all views
+    uint32_t key_bits = 0;     // 24 depth bits + the tile bits (the reference's pair keys)
+    uint32_t strip_bits = 0;   // bits of a strip number
+    uint32_t strip_passes = 0;
+    uint32_t entry_cap = 0;    // strip entries the binning holds
+    uint32_t seg_cap = 0;      // segments: entry_cap / kStripSeg + a partial one a strip
+    // A frame of several views whose ranks are grouped by view (the view
+    // pass), so that each view's strip entries are one run: its strip sort
+    // orders each run by the view's own strip number (launch_segment_sort),
+    // view_strip_bits bits; the sort's counts are sized for entry_pad more
+    // entries (a partial partition a view).
+    bool segmented = false;
+    uint32_t view_strip_bits = 0;
+    uint32_t entry_pad = 0;
+    uint32_t capacity = 0;     // pairs the pair buffer holds
+    std::vector<uint32_t> bases;  // each instance's first Gaussian in a view's slots, then count
+    bool matte = false, traced = false, under = false;  // the walk's variants (athx_targets)
+    // The plain walk reads the strip entries themselves and no pairs are
+    // listed (their readers list them on request: list_pairs): a plain frame
+    // whose targets keep no walk for the adjoint, its masks in the keys, its
+    // tiles 16 or 32 pixels.
+    bool direct = false;
+    bool variants() const { return matte || traced || under; }
+};
+
 }  // namespace
 
 struct athx_ctx {
@@ -94,6 +126,7 @@ struct athx_ctx {
     // masks and the per (tile, segment) table.
     DeviceBuffer strip_keys, strip_slots, strip_alt_keys, strip_alt_slots, strip_sort_meta;
     DeviceBuffer strip_ranges, segbase, seg_map, masks, seg_table, rank_fp;
+    DeviceBuffer tally;  // the emission's pair words (kTallyWords) of a frame that lists no pairs
     // For the frame's readers: exact tile counts and their scan in depth order.
     DeviceBuffer exact, exact_offsets, exact_status;
     DeviceBuffer api_sort_meta, api_alt_keys, api_alt_vals, api_scan_status, api_count;
@@ -113,6 +146,9 @@ struct athx_ctx {
     uint32_t last_instances = 0;  // the clouds the last frame projected (athx_render_instances)
     bool last_under = false;      // the last frame's walks ended at an under layer
     bool last_sorted_in_alt = false;  // the ranked slots are in depth_alt_slots
+    bool last_strips_in_alt = false;  // the sorted strip entries are in the strip_alt buffers
+    FrameShape last_shape;            // the sizes the last frame ran at
+    bool pairs_listed = true;         // its pairs and ranges are in pair_vals and ranges (list_pairs)
     // The last frame sorted each view's slots apart (its ranks grouped by
     // view): the exact offsets, scanned in the frame's whole depth order,
     // then sort that order on request (order_* buffers).
@@ -162,7 +198,7 @@ std::vector<DeviceBuffer*> all_buffers(athx_ctx* ctx) {
             &ctx->strip_keys, &ctx->strip_slots, &ctx->strip_alt_keys, &ctx->strip_alt_slots, &ctx->strip_sort_meta,
             &ctx->segments, &ctx->depth_segments, &ctx->order_keys, &ctx->order_slots, &ctx->order_alt_keys,
             &ctx->order_alt_slots, &ctx->order_meta,
-            &ctx->strip_ranges, &ctx->segbase, &ctx->seg_map, &ctx->rank_fp, &ctx->masks, &ctx->seg_table, &ctx->exact, &ctx->exact_offsets,
+            &ctx->strip_ranges, &ctx->segbase, &ctx->seg_map, &ctx->rank_fp, &ctx->tally, &ctx->masks, &ctx->seg_table, &ctx->exact, &ctx->exact_offsets,
             &ctx->exact_status, &ctx->api_sort_meta, &ctx->api_alt_keys, &ctx->api_alt_vals, &ctx->api_scan_status,
             &ctx->api_count, &ctx->ingest_keep, &ctx->ingest_dest, &ctx->ingest_total, &ctx->ref_records,
             &ctx->ref_keys, &ctx->ref_values, &ctx->ref_alt_keys, &ctx->ref_alt_values, &ctx->ref_sort_meta,
@@ -557,33 +593,6 @@ SortScratch sort_scratch(const DeviceBuffer& meta, void* alt_keys, uint32_t* alt
     return sc;
 }
 
-// The sizes a frame runs at.
-struct FrameShape {
-    uint32_t nviews = 0;
-    uint32_t instances = 1;    // clouds projected into each view
-    uint32_t count = 0;        // Gaussians a view: every instance's, back to back
-    uint32_t slots = 0;        // views * count
-    uint32_t tiles = 0;        // over all views
-    uint32_t strips = 0;       // over all views
-    uint32_t key_bits = 0;     // 24 depth bits + the tile bits (the reference's pair keys)
-    uint32_t strip_bits = 0;   // bits of a strip number
-    uint32_t strip_passes = 0;
-    uint32_t entry_cap = 0;    // strip entries the binning holds
-    uint32_t seg_cap = 0;      // segments: entry_cap / kStripSeg + a partial one a strip
-    // A frame of several views whose ranks are grouped by view (the view
-    // pass), so that each view's strip entries are one run: its strip sort
-    // orders each run by the view's own strip number (launch_segment_sort),
-    // view_strip_bits bits; the sort's counts are sized for entry_pad more
-    // entries (a partial partition a view).
-    bool segmented = false;
-    uint32_t view_strip_bits = 0;
-    uint32_t entry_pad = 0;
-    uint32_t capacity = 0;     // pairs the pair buffer holds
-    std::vector<uint32_t> bases;  // each instance's first Gaussian in a view's slots, then count
-    bool matte = false, traced = false, under = false;  // the walk's variants (athx_targets)
-    bool variants() const { return matte || traced || under; }
-};
-
 bool masks_in_keys(const FrameShape& fs) { return fs.strip_bits <= 16; }
 // The segmented strip sort's partitions: the entries' and a partial one a view.
 uint32_t segment_parts_cap(const FrameShape& fs) { return div_up(fs.entry_cap, kSegmentPart) + fs.nviews; }
@@ -657,6 +666,11 @@ athx_status begin_frame(athx_ctx* ctx, const athx_view* views, uint32_t nviews, 
     }
     fs.view_strip_bits = bits_for(view_strips);
     fs.segmented = grouped_by_view(fs) && masks_in_keys(fs) && nviews <= kMaxSegmentViews;
+    bool kept = false;  // the adjoint walks the pairs back from targets[].last
+    for (uint32_t k = 0; k < nviews; ++k) {
+        kept = kept || targets[k].last != nullptr;
+    }
+    fs.direct = !kept && !fs.variants() && masks_in_keys(fs) && settings->tile != 8 && fs.slots != 0;
     return ATHX_OK;
 }
 
@@ -685,7 +699,10 @@ athx_status reserve_front(athx_ctx* ctx, const FrameShape& fs) {
     }
     ATHX_HIP(ctx, reserve(ctx, ctx->strip_ranges, (size_t)fs.strips * 8 + 16), "strip ranges");
     ATHX_HIP(ctx, reserve(ctx, ctx->segbase, (size_t)fs.strips * 4 + 16), "strip segments");
-    ATHX_HIP(ctx, reserve(ctx, ctx->rank_fp, slots * 32 + 32), "ranked footprints");
+    if (!masks_in_keys(fs)) {
+        ATHX_HIP(ctx, reserve(ctx, ctx->rank_fp, slots * 32 + 32), "ranked footprints");
+    }
+    ATHX_HIP(ctx, reserve(ctx, ctx->tally, (size_t)kTallyWords * kTallyStride * 8), "pair tally");
     if (fs.matte) {
         ATHX_HIP(ctx, reserve(ctx, ctx->slot_ids, slots * 4 + 16), "Cryptomatte ids");
     }
@@ -695,9 +712,9 @@ athx_status reserve_front(athx_ctx* ctx, const FrameShape& fs) {
 // The binning's buffers for fs.entry_cap entries.
 athx_status reserve_bins(athx_ctx* ctx, const FrameShape& fs) {
     const size_t cap = fs.entry_cap;
-    ATHX_HIP(ctx, reserve(ctx, ctx->strip_keys, cap * 4 + 16), "strip keys");
+    ATHX_HIP(ctx, reserve(ctx, ctx->strip_keys, cap * 4 + 32), "strip keys");
     ATHX_HIP(ctx, reserve(ctx, ctx->strip_slots, cap * 4 + 16), "strip slots");
-    ATHX_HIP(ctx, reserve(ctx, ctx->strip_alt_keys, cap * 4 + 16), "strip sort keys");
+    ATHX_HIP(ctx, reserve(ctx, ctx->strip_alt_keys, cap * 4 + 32), "strip sort keys");
     ATHX_HIP(ctx, reserve(ctx, ctx->strip_alt_slots, cap * 4 + 16), "strip sort slots");
     const uint32_t passes = fs.segmented ? div_up(fs.view_strip_bits, 8) : fs.strip_passes;
     ATHX_HIP(ctx, reserve(ctx, ctx->strip_sort_meta, sort_meta_words(fs.entry_cap + fs.entry_pad, passes) * 4 + 16),
@@ -706,7 +723,7 @@ athx_status reserve_bins(athx_ctx* ctx, const FrameShape& fs) {
         ATHX_HIP(ctx, reserve(ctx, ctx->segments, ((size_t)segment_parts_cap(fs) + 4u * fs.nviews + 4) * 4),
                  "strip segments");
     }
-    ATHX_HIP(ctx, reserve(ctx, ctx->masks, cap * 2 + 16), "entry masks");
+    ATHX_HIP(ctx, reserve(ctx, ctx->masks, cap * 2 + 32), "entry masks");
     ATHX_HIP(ctx, reserve(ctx, ctx->seg_map, (size_t)fs.seg_cap * 32 + 32), "segment descriptors");
     const size_t table = (size_t)kStripTiles * fs.seg_cap;
     // The table's scan status follows the table.
@@ -716,6 +733,9 @@ athx_status reserve_bins(athx_ctx* ctx, const FrameShape& fs) {
 }
 
 athx_status reserve_pairs(athx_ctx* ctx, const FrameShape& fs) {
+    if (fs.direct) {
+        return ATHX_OK;
+    }
     ATHX_HIP(ctx, reserve(ctx, ctx->pair_vals, (size_t)fs.capacity * 4 + 16), "pair values");
     return ATHX_OK;
 }
@@ -839,7 +859,8 @@ athx_status enqueue_front(athx_ctx* ctx, const std::vector<ProjectArgs>& pas, co
     const uint32_t tile = pas.empty() ? 16u : pas[0].tile;
     ATHX_HIP(ctx, launch_settle_count(as<DView>(ctx->views), fs.count, tile, fs.slots, as<float>(ctx->records),
                                       as<uint32_t>(ctx->touched), as<uint32_t>(ctx->depth_keys),
-                                      reinterpret_cast<uint64_t*>(ctx->scan_status.ptr), s),
+                                      reinterpret_cast<uint64_t*>(ctx->scan_status.ptr), s,
+                                      fs.direct ? as<uint64_t>(ctx->tally) : nullptr),
              "settle");
     // Several views: each view's visible slots are sorted apart, so the
     // ranks come out grouped by view, each view's in depth order. A strip is
@@ -947,14 +968,19 @@ athx_status enqueue_segments(athx_ctx* ctx, const FrameShape& fs, hipStream_t s)
     return ATHX_OK;
 }
 
-// The strip entries, emitted in depth order, sorted on the strip, their
-// segments scanned, tested and counted, and the counts scanned: the pair
+athx_status enqueue_segment_counts(athx_ctx* ctx, const FrameShape& fs, uint32_t n, uint32_t tile, hipStream_t s,
+                                   bool strips_in_alt);
+
+// The strip entries, emitted in depth order, sorted on the strip and, unless
+// the frame lists no pairs (fs.direct: the emission's tally is the total),
+// their segments counted (enqueue_segment_counts): the pair
 // total lands in totals[kTotalPairs]. Every count is read on the device
 // and bounded by fs's capacities, so the launches can be captured.
 athx_status enqueue_bins(athx_ctx* ctx, const FrameShape& fs, uint32_t n, uint32_t tile, hipStream_t s, bool timed,
                          bool& strips_in_alt, bool count = false) {
     uint64_t* totals = as<uint64_t>(ctx->totals);
     const bool masked = masks_in_keys(fs);
+    uint64_t* tally = fs.direct ? as<uint64_t>(ctx->tally) : nullptr;
     if (masked) {
         // Counting frames keep each rank's tiles (its entries' mask bits) for the counters.
         uint32_t* rank_tiles = nullptr;
@@ -967,7 +993,7 @@ athx_status enqueue_bins(athx_ctx* ctx, const FrameShape& fs, uint32_t n, uint32
                                              sorted_slots_of(ctx, ctx->last_sorted_in_alt), as<uint32_t>(ctx->offsets),
                                              totals + kTotalVisible, fs.slots, fs.entry_cap, as<float>(ctx->records),
                                              as<uint32_t>(ctx->strip_keys), as<uint32_t>(ctx->strip_slots), rank_tiles,
-                                             s, fs.segmented ? view_entry_of(ctx, fs) : nullptr),
+                                             s, fs.segmented ? view_entry_of(ctx, fs) : nullptr, tally),
                  "strip entries");
         if (fs.segmented) {
             if (athx_status st = enqueue_segments(ctx, fs, s); st != ATHX_OK) {
@@ -993,7 +1019,8 @@ athx_status enqueue_bins(athx_ctx* ctx, const FrameShape& fs, uint32_t n, uint32
     if (segmented) {
         ATHX_HIP(ctx, launch_segment_sort(as<uint32_t>(ctx->strip_keys), as<uint32_t>(ctx->strip_slots),
                                           segments_of(ctx, fs), segment_parts_cap(fs), fs.view_strip_bits, sc, s,
-                                          strips_in_alt, true, mask_sort ? as<uint16_t>(ctx->masks) : nullptr),
+                                          strips_in_alt, true,
+                                          mask_sort || fs.direct ? as<uint16_t>(ctx->masks) : nullptr),
                  "strip sort");
     } else {
         ATHX_HIP(ctx, launch_sort(as<uint32_t>(ctx->strip_keys), as<uint32_t>(ctx->strip_slots),
@@ -1007,21 +1034,31 @@ athx_status enqueue_bins(athx_ctx* ctx, const FrameShape& fs, uint32_t n, uint32
         ATHX_HIP(ctx, launch_strip_ranges_seg(sc.offsets, segments_of(ctx, fs), fs.nviews,
                                               as<uint32_t>(ctx->tile_bases) + fs.nviews + 1, fs.strips,
                                               1u << fs.view_strip_bits, totals + kTotalBinned,
-                                              as<uint32_t>(ctx->strip_ranges), s),
+                                              as<uint32_t>(ctx->strip_ranges), s, tally, totals + kTotalPairs),
                  "strip ranges");
     } else {
         ATHX_HIP(ctx, launch_ranges(keys, totals + (segmented ? kTotalBinned : kTotalEntries), fs.entry_cap,
-                                    fs.strips, as<uint32_t>(ctx->strip_ranges), s, masked ? 0xFFFFu : ~0u),
+                                    fs.strips, as<uint32_t>(ctx->strip_ranges), s, masked ? 0xFFFFu : ~0u, tally,
+                                    totals + kTotalPairs),
                  "strip ranges");
     }
+    if (timed) {
+        ATHX_HIP(ctx, hipEventRecord(ctx->ev[4], s), "event");
+    }
+    return fs.direct ? ATHX_OK : enqueue_segment_counts(ctx, fs, n, tile, s, strips_in_alt);
+}
+
+// The sorted entries cut into segments, tested and counted, and the counts
+// scanned: the pair total lands in totals[kTotalPairs] and every (tile,
+// segment)'s first pair in the table.
+athx_status enqueue_segment_counts(athx_ctx* ctx, const FrameShape& fs, uint32_t n, uint32_t tile, hipStream_t s,
+                                   bool strips_in_alt) {
+    uint64_t* totals = as<uint64_t>(ctx->totals);
     ATHX_HIP(ctx, launch_seg_scan(as<uint32_t>(ctx->strip_ranges), fs.strips, as<uint32_t>(ctx->segbase),
                                   totals + kTotalSegs, as<uint32_t>(ctx->scan_status), s),
              "segments");
     const StripBins b = bins_of(ctx, fs, n, tile, strips_in_alt);
     ATHX_HIP(ctx, launch_seg_desc(b, as<uint4>(ctx->seg_map), s), "segment descriptors");
-    if (timed) {
-        ATHX_HIP(ctx, hipEventRecord(ctx->ev[4], s), "event");
-    }
     ATHX_HIP(ctx, launch_strip_count(b, s), "strip counts");
     uint32_t* table = as<uint32_t>(ctx->seg_table);
     uint32_t* table_status = table + (size_t)kStripTiles * fs.seg_cap;
@@ -1035,20 +1072,33 @@ athx_status enqueue_bins(athx_ctx* ctx, const FrameShape& fs, uint32_t n, uint32
 athx_status enqueue_draw(athx_ctx* ctx, const FrameShape& fs, const athx_settings* settings, hipStream_t s,
                          bool timed, bool strips_in_alt, bool capturing = false) {
     const StripBins b = bins_of(ctx, fs, fs.count, settings->tile, strips_in_alt);
-    ATHX_HIP(ctx, launch_strip_pairs(b, s), "pairs");
+    ctx->last_strips_in_alt = strips_in_alt;
+    if (!fs.direct) {
+        ATHX_HIP(ctx, launch_strip_pairs(b, s), "pairs");
+    }
     if (timed) {
         ATHX_HIP(ctx, hipEventRecord(ctx->ev[5], s), "event");
     }
-    ATHX_HIP(ctx, launch_tile_ranges(b, as<uint32_t>(ctx->tile_bases), fs.tiles, as<uint32_t>(ctx->ranges), s),
-             "ranges");
+    if (!fs.direct) {
+        ATHX_HIP(ctx, launch_tile_ranges(b, as<uint32_t>(ctx->tile_bases), fs.tiles, as<uint32_t>(ctx->ranges), s),
+                 "ranges");
+    }
     if (timed) {
         ATHX_HIP(ctx, hipEventRecord(ctx->ev[6], s), "event");
     }
-    ATHX_HIP(ctx, launch_blend(as<DView>(ctx->views), as<uint32_t>(ctx->tile_bases), fs.nviews, fs.tiles,
+    if (fs.direct) {
+        const EntryWalk entries{b.strip_ranges, b.strip_keys, fs.segmented ? b.masks : nullptr, b.strip_slots};
+        ATHX_HIP(ctx, launch_blend_entries(as<DView>(ctx->views), as<uint32_t>(ctx->tile_bases), fs.nviews, fs.tiles,
+                                           settings->tile, entries, as<float>(ctx->records), settings->depth_mode,
+                                           settings->depth_threshold, s),
+                 "blend");
+    } else {
+        ATHX_HIP(ctx, launch_blend(as<DView>(ctx->views), as<uint32_t>(ctx->tile_bases), fs.nviews, fs.tiles,
                                settings->tile, settings->batch, as<uint32_t>(ctx->ranges), as<uint32_t>(ctx->pair_vals),
                                as<float>(ctx->records), settings->depth_mode, settings->depth_threshold, s,
                                fs.variants(), fs.matte ? as<uint32_t>(ctx->slot_ids) : nullptr),
-             "blend");
+                 "blend");
+    }
     if (timed) {
         ATHX_HIP(ctx, hipEventRecord(ctx->ev[7], s), "event");
     }
@@ -1125,8 +1175,34 @@ void finish_frame(athx_ctx* ctx, const athx_settings* settings, const FrameShape
     ctx->last_entry_cap = fs.entry_cap;
     ctx->last_key_bits = fs.key_bits;
     ctx->last_true_pairs = pairs_known;
+    ctx->last_shape = fs;
+    ctx->pairs_listed = !fs.direct;
     ctx->have_frame = true;
     ctx->serial += 1;
+}
+
+// The last frame's pairs and ranges for their readers (the adjoint, the
+// contributions, copy_frame), where the frame listed none: from the sorted
+// entries it left, up to its capacity as the frame itself would have.
+athx_status list_pairs(athx_ctx* ctx, hipStream_t s) {
+    if (ctx->pairs_listed) {
+        return ATHX_OK;
+    }
+    FrameShape fs = ctx->last_shape;
+    fs.direct = false;
+    if (athx_status st = reserve_pairs(ctx, fs); st != ATHX_OK) {
+        return st;
+    }
+    if (athx_status st = enqueue_segment_counts(ctx, fs, fs.count, ctx->last_tile, s, ctx->last_strips_in_alt);
+        st != ATHX_OK) {
+        return st;
+    }
+    const StripBins b = bins_of(ctx, fs, fs.count, ctx->last_tile, ctx->last_strips_in_alt);
+    ATHX_HIP(ctx, launch_strip_pairs(b, s), "pairs");
+    ATHX_HIP(ctx, launch_tile_ranges(b, as<uint32_t>(ctx->tile_bases), fs.tiles, as<uint32_t>(ctx->ranges), s),
+             "ranges");
+    ctx->pairs_listed = true;
+    return ATHX_OK;
 }
 
 // The frame a backward pass or a contribution walk names must be the one
@@ -1353,7 +1429,7 @@ athx_status render_frame(athx_ctx* ctx, const athx_view* views, uint32_t nviews,
         if (athx_status st = read_totals(ctx, s); st != ATHX_OK) {
             return st;
         }
-        fitted = host[kTotalEntries] <= fs.entry_cap && host[kTotalPairs] <= fs.capacity;
+        fitted = host[kTotalEntries] <= fs.entry_cap && (fs.direct || host[kTotalPairs] <= fs.capacity);
     } else if (athx_status st = read_totals(ctx, s); st != ATHX_OK) {
         return st;
     }
@@ -1367,6 +1443,11 @@ athx_status render_frame(athx_ctx* ctx, const athx_view* views, uint32_t nviews,
             set_entry_cap(fs, std::max<uint32_t>((uint32_t)entries, 1u));
             if (athx_status st = reserve_bins(ctx, fs); st != ATHX_OK) {
                 return st;
+            }
+            if (ahead && fs.direct) {
+                // The emission that did not fit has tallied its pairs already.
+                ATHX_HIP(ctx, launch_fill_u32(as<uint32_t>(ctx->tally), 0u, 2u * kTallyWords * kTallyStride, s),
+                         "clear the pair tally");
             }
             if (athx_status st = enqueue_bins(ctx, fs, fs.count, settings->tile, s, timed, strips_in_alt, settings->count_splats != 0); st != ATHX_OK) {
                 return st;
@@ -1396,6 +1477,13 @@ athx_status render_frame(athx_ctx* ctx, const athx_view* views, uint32_t nviews,
         ATHX_HIP(ctx, hipStreamSynchronize(s), "wait for the counted frame");
     }
     const uint64_t pairs64 = host[kTotalPairs];
+    if (fs.direct) {
+        // No pair buffer bounds the frame; its readers' would be this large.
+        if (pairs64 >= kMaxPairs) {
+            return fail(ctx, ATHX_UNSUPPORTED, "more than 2^30 (tile, Gaussian) pairs in one frame");
+        }
+        fs.capacity = std::max<uint32_t>((uint32_t)pairs64, 1u);
+    }
     ctx->entry_last = std::min<uint64_t>(grown(host[kTotalEntries]), kMaxPairs - 1);
     ctx->pair_last = std::min<uint64_t>(grown(pairs64), kMaxPairs - 1);
     ctx->entry_hint = std::max(ctx->entry_hint, ctx->entry_last);
@@ -1608,6 +1696,9 @@ ATHX_API athx_status athx_render_backward(athx_ctx* ctx, const athx_view* views,
     if (athx_status st = upload_views(ctx, nviews, s); st != ATHX_OK) {
         return st;
     }
+    if (athx_status st = list_pairs(ctx, s); st != ATHX_OK) {
+        return st;
+    }
     const uint32_t slots = gaussians->count * nviews;
     ATHX_HIP(ctx, reserve(ctx, ctx->grad2d, (size_t)slots * kGrad2d * sizeof(float) + 16), "2D gradients");
     return enqueue_backward(ctx, project_args(gaussians, settings), nviews, slots, settings, *grads, s);
@@ -1662,6 +1753,9 @@ ATHX_API athx_status athx_contribution(athx_ctx* ctx, const athx_view* views, ui
         return fail(ctx, ATHX_INVALID_ARGUMENT, "the views differ from the rendered frame's");
     }
     if (athx_status st = upload_views(ctx, nviews, s); st != ATHX_OK) {
+        return st;
+    }
+    if (athx_status st = list_pairs(ctx, s); st != ATHX_OK) {
         return st;
     }
     const uint64_t words = (uint64_t)ctx->last_n * nviews * (mode == 4 ? 4u : mode == 1 ? 1u : 2u);
@@ -1780,6 +1874,12 @@ ATHX_API athx_status athx_copy_frame(athx_ctx* ctx, athx_frame_part part, void* 
     }
     ATHX_HIP(ctx, hipSetDevice(ctx->device), "set device");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (part == ATHX_PART_PAIR_KEYS || part == ATHX_PART_PAIR_VALUES || part == ATHX_PART_RANGES) {
+        if (athx_status st = list_pairs(ctx, s); st != ATHX_OK) {
+            return st;
+        }
+        src = part == ATHX_PART_PAIR_VALUES ? ctx->pair_vals.ptr : ctx->ranges.ptr;
+    }
     if (part == ATHX_PART_PAIR_KEYS) {
         ATHX_HIP(ctx, launch_pair_keys(as<uint32_t>(ctx->ranges), ctx->last_tiles, as<uint32_t>(ctx->pair_vals),
                                        as<uint32_t>(ctx->depth_keys), static_cast<uint64_t*>(dst), s),

@@ -784,7 +784,9 @@ __device__ inline uint32_t lower_bound_tile(const uint32_t* tiles, uint32_t n, u
 __global__ void __launch_bounds__(256) ranges_kernel(const uint32_t* __restrict__ keys,
                                                      const uint64_t* __restrict__ n_dev, uint32_t cap, uint32_t tiles,
                                                      uint32_t key_mask,
-                                                     uint32_t* __restrict__ ranges) {
+                                                     uint32_t* __restrict__ ranges, const uint64_t* __restrict__ tally,
+                                                     uint64_t* __restrict__ pair_total) {
+    sum_tally(tally, pair_total);
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= tiles) {
         return;
@@ -812,8 +814,13 @@ template <uint32_t kSettleThreads>
 __global__ void __launch_bounds__(kSettleThreads) settle_count_kernel(const DView* __restrict__ views, uint32_t n, uint32_t T,
                                                            uint32_t slots, const float* __restrict__ records,
                                                            uint32_t* __restrict__ touched, uint32_t* __restrict__ keys,
-                                                           uint64_t* __restrict__ sums) {
+                                                           uint64_t* __restrict__ sums, uint64_t* __restrict__ tally) {
     __shared__ uint32_t s_wave[kSettleThreads / 64];
+    if (tally && blockIdx.x == 0) {
+        for (uint32_t w = threadIdx.x; w < kTallyWords; w += kSettleThreads) {
+            tally[w * kTallyStride] = 0;
+        }
+    }
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t first_block = (uint64_t)blockIdx.x * kCompactTile;
     constexpr uint32_t kPer = kCompactTile / kSettleThreads;
@@ -1094,7 +1101,8 @@ __global__ void __launch_bounds__(kEmitThreads) strip_mask_emit_kernel(const DVi
                                                                        uint32_t* __restrict__ keys_out,
                                                                        uint32_t* __restrict__ slots_out,
                                                                        uint32_t* __restrict__ rank_tiles,
-                                                                       uint32_t* __restrict__ view_entry) {
+                                                                       uint32_t* __restrict__ view_entry,
+                                                                       uint64_t* __restrict__ tally) {
     __shared__ uint32_t s_end[kEmitThreads];
     __shared__ uint32_t s_tiles[kEmitThreads]; // rank: tiles its entries' masks hold (counting frames)
     __shared__ float4 s_geo[kEmitThreads];   // rank: centre x, y, conic a, b
@@ -1157,7 +1165,7 @@ __global__ void __launch_bounds__(kEmitThreads) strip_mask_emit_kernel(const DVi
     // step), and a running max over the positions carries each mark on to
     // the run's end; a step that starts inside a run continues the last
     // step's final rank.
-    uint32_t carried = 0;
+    uint32_t carried = 0, pairs = 0;
     for (uint32_t g0 = 0, step = 0; g0 < total; g0 += 64, ++step) {
         if (count != 0 && start >= g0 && start < g0 + 64u) {
             s_own[wbase + (start - g0)] = (step << 8) | (lane + 1u);
@@ -1212,8 +1220,17 @@ __global__ void __launch_bounds__(kEmitThreads) strip_mask_emit_kernel(const DVi
             keys_out[at] = (I.w + __umul24(row, strips_x) + sxi) | (mask << 16);
             slots_out[at] = I.x;
         }
+        const uint32_t here = (uint32_t)__builtin_popcount(mask);
+        pairs += here;
         if (rank_tiles) {
-            atomicAdd(&s_tiles[wbase + j], (uint32_t)__builtin_popcount(mask));
+            atomicAdd(&s_tiles[wbase + j], here);
+        }
+    }
+    if (tally) {
+        const uint32_t sum = wave_inclusive_sum_dpp(pairs);
+        if (lane == 63 && sum != 0) {
+            const uint32_t word = (blockIdx.x * (kEmitThreads / 64) + (threadIdx.x >> 6)) % kTallyWords;
+            atomicAdd(reinterpret_cast<unsigned long long*>(tally + word * kTallyStride), (unsigned long long)sum);
         }
     }
     if (rank_tiles && k < visible) {
@@ -1750,16 +1767,17 @@ hipError_t launch_project(const ProjectArgs& a, const DView* views_dev, uint32_t
 }
 
 hipError_t launch_settle_count(const DView* views_dev, uint32_t n, uint32_t tile, uint32_t slots, const float* records,
-                               uint32_t* touched, uint32_t* depth_keys, uint64_t* sums, hipStream_t s) {
+                               uint32_t* touched, uint32_t* depth_keys, uint64_t* sums, hipStream_t s,
+                               uint64_t* tally) {
     if (slots == 0) {
         return hipSuccess;
     }
     if (slots >= kSettleWide) {
         hipLaunchKernelGGL(settle_count_kernel<256>, dim3(div_up(slots, kCompactTile)), dim3(256), 0, s, views_dev, n,
-                           tile, slots, records, touched, depth_keys, sums);
+                           tile, slots, records, touched, depth_keys, sums, tally);
     } else {
         hipLaunchKernelGGL(settle_count_kernel<1024>, dim3(div_up(slots, kCompactTile)), dim3(1024), 0, s, views_dev,
-                           n, tile, slots, records, touched, depth_keys, sums);
+                           n, tile, slots, records, touched, depth_keys, sums, tally);
     }
     return hipGetLastError();
 }
@@ -1799,12 +1817,13 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t 
 }
 
 hipError_t launch_ranges(const uint32_t* sorted_keys, const uint64_t* n_dev, uint32_t cap, uint32_t tiles,
-                         uint32_t* ranges, hipStream_t s, uint32_t key_mask) {
+                         uint32_t* ranges, hipStream_t s, uint32_t key_mask, const uint64_t* tally,
+                         uint64_t* pair_total) {
     if (tiles == 0) {
         return hipSuccess;
     }
     hipLaunchKernelGGL(ranges_kernel, dim3(div_up(tiles, 256)), dim3(256), 0, s, sorted_keys, n_dev, cap, tiles,
-                       key_mask, ranges);
+                       key_mask, ranges, tally, pair_total);
     return hipGetLastError();
 }
 
@@ -1858,13 +1877,13 @@ hipError_t launch_strip_count(const StripBins& b, hipStream_t s) {
 hipError_t launch_strip_mask_emit(const DView* views_dev, uint32_t n, uint32_t tile, const uint32_t* sorted_slots,
                                   const uint32_t* offsets, const uint64_t* visible_dev, uint32_t max_visible,
                                   uint32_t cap, const float* records, uint32_t* strip_keys, uint32_t* strip_slots,
-                                  uint32_t* rank_tiles, hipStream_t s, uint32_t* view_entry) {
+                                  uint32_t* rank_tiles, hipStream_t s, uint32_t* view_entry, uint64_t* tally) {
     if (max_visible == 0 || cap == 0) {
         return hipSuccess;
     }
     hipLaunchKernelGGL(strip_mask_emit_kernel, dim3(div_up(max_visible, kEmitThreads)), dim3(kEmitThreads), 0, s,
                        views_dev, n, tile, sorted_slots, offsets, visible_dev, max_visible, cap, records,
-                       strip_keys, strip_slots, rank_tiles, view_entry);
+                       strip_keys, strip_slots, rank_tiles, view_entry, tally);
     return hipGetLastError();
 }
 

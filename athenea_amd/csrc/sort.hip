@@ -477,7 +477,7 @@ __global__ void __launch_bounds__(kT) downsweep_kernel(const K* __restrict__ kin
                                                        K* __restrict__ kout, uint32_t* __restrict__ vout, L layout,
                                                        D digit, uint32_t width,
                                                        const uint32_t* __restrict__ offsets,
-                                                       uint16_t* __restrict__ mout) {
+                                                       uint16_t* __restrict__ mout, uint32_t keep_keys) {
     static_assert(kT >= kRadix && kT % 64 == 0, "a thread a digit");
     constexpr uint32_t kW = kT / 64;
     constexpr uint32_t kP = kT * kItems;
@@ -562,11 +562,13 @@ __global__ void __launch_bounds__(kT) downsweep_kernel(const K* __restrict__ kin
         const uint32_t v = s_vals[i];
         const uint32_t dk = digit(k, v, pt.base);
         const uint32_t dst = s_digit_base[dk] + (i - s_block_start[dk]);
-        // mout: a strip sort's last pass keeps only each key's upper half
-        // (its tile mask); the strips' runs come from the counts instead.
+        // mout: a strip sort's last pass writes each key's upper half (its
+        // tile mask) apart; a sort of one pass keeps nothing else (the
+        // strips' runs come from the counts), a longer one the keys too.
         if (mout) {
             mout[dst] = (uint16_t)((uint32_t)k >> 16);
-        } else {
+        }
+        if (keep_keys != 0) {
             kout[dst] = k;
         }
         vout[dst] = v;
@@ -650,7 +652,7 @@ hipError_t sort_impl(K* keys, uint32_t* values, const uint64_t* n_dev, uint32_t 
                 return e;
             }
             hipLaunchKernelGGL((downsweep_kernel<K, KeyDigit, kT, PlainLayout>), dim3(rparts), dim3(kT), 0, s, kin,
-                               vin, kout, vout, layout, digit, width, sc.offsets, nullptr);
+                               vin, kout, vout, layout, digit, width, sc.offsets, nullptr, 1u);
             K* tk = kin; kin = kout; kout = tk;
             uint32_t* tv = vin; vin = vout; vout = tv;
         }
@@ -738,7 +740,8 @@ hipError_t segment_passes(uint32_t* keys, uint32_t* values, const SegmentArgs& g
             return e;
         }
         hipLaunchKernelGGL((downsweep_kernel<uint32_t, D, kT, SegLayout>), dim3(parts), dim3(kT), 0, s, kin, vin,
-                           kout, vout, layout, digit, width, sc.offsets, p + 1 == passes ? mask_out : nullptr);
+                           kout, vout, layout, digit, width, sc.offsets, p + 1 == passes ? mask_out : nullptr,
+                           mask_out && passes == 1 ? 0u : 1u);
         in_alt = !in_alt;
     }
     return hipGetLastError();
@@ -768,7 +771,10 @@ __global__ void __launch_bounds__(256) strip_ranges_seg_kernel(const uint32_t* _
                                                                uint32_t nviews, const uint32_t* __restrict__ strip_bases,
                                                                uint32_t strips, uint32_t radix,
                                                                const uint64_t* __restrict__ total_dev,
-                                                               uint32_t* __restrict__ ranges) {
+                                                               uint32_t* __restrict__ ranges,
+                                                               const uint64_t* __restrict__ tally,
+                                                               uint64_t* __restrict__ pair_total) {
+    sum_tally(tally, pair_total);
     const uint32_t st = blockIdx.x * blockDim.x + threadIdx.x;
     if (st >= strips) {
         return;
@@ -800,12 +806,13 @@ __global__ void __launch_bounds__(256) strip_ranges_seg_kernel(const uint32_t* _
 
 hipError_t launch_strip_ranges_seg(const uint32_t* offsets, const SegmentArgs& g, uint32_t nviews,
                                    const uint32_t* strip_bases, uint32_t strips, uint32_t radix,
-                                   const uint64_t* total_dev, uint32_t* ranges, hipStream_t s) {
+                                   const uint64_t* total_dev, uint32_t* ranges, hipStream_t s, const uint64_t* tally,
+                                   uint64_t* pair_total) {
     if (strips == 0) {
         return hipSuccess;
     }
     hipLaunchKernelGGL(strip_ranges_seg_kernel, dim3(div_up(strips, 256)), dim3(256), 0, s, offsets, g, nviews,
-                       strip_bases, strips, radix, total_dev, ranges);
+                       strip_bases, strips, radix, total_dev, ranges, tally, pair_total);
     return hipGetLastError();
 }
 

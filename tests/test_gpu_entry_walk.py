@@ -1,0 +1,111 @@
+"""Frames whose targets keep no walk are blended straight from the strip
+entries, with no pairs listed: the same image as the walk over listed pairs bit
+for bit, the same pair total, and the pairs, ranges, contributions and
+gradients still there for who asks afterwards. Sizes: tiles of 16 and 32 in
+ragged pictures (strips cut short), strips of no entry and of many fills, one
+view (masks in the keys), several (masks apart, one- and two-pass strip sorts),
+and a frame that outgrows the entries the frame before it left room for."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from athenea_amd import RenderSettings, TileRasterizer, camera, synthetic
+from athenea_amd.raster import GaussianCloud
+
+pytestmark = pytest.mark.gpu
+
+PARTS = ("pair_keys", "pair_values", "ranges")
+
+
+@pytest.fixture
+def raster():
+    r = TileRasterizer(0)
+    yield r
+    r.close()
+
+
+def a_view(width, height, azimuth=0.0, radius=3.0):
+    cam = camera.orbit_camera(radius, azimuth, 60.0)
+    cam.lens.near_z = 0.01
+    return camera.view_for(cam, width, height)
+
+
+def both(raster, cloud, views, settings):
+    """The frame with its pairs listed, then the one without."""
+    kept, kept_stats = raster.render(views, cloud, settings, keep_backward=True)
+    kept_bufs = raster.frame_buffers()
+    plain, stats = raster.render(views, cloud, settings)
+    assert stats.pairs == kept_stats.pairs and stats.visible == kept_stats.visible
+    for a, b in zip(kept, plain):
+        assert torch.equal(a.colour, b.colour) and torch.equal(a.depth, b.depth)
+    bufs = raster.frame_buffers()
+    for part in PARTS:
+        assert torch.equal(kept_bufs[part], bufs[part]), part
+    return kept, stats
+
+
+@pytest.mark.parametrize("tile", [16, 32])
+@pytest.mark.parametrize("depth", ["mean", "threshold"])
+@pytest.mark.parametrize("n,size", [(1, (3, 2)), (700, (250, 37)), (60000, (530, 131))])
+def test_one_view(raster, tile, depth, n, size):
+    print("entry walk", tile, depth, n, size, flush=True)
+    cloud = GaussianCloud.from_numpy(synthetic.make_cloud(n, 5, log_scale_mean=-4.0, axis_spread=0.7), "cuda:0")
+    both(raster, cloud, [a_view(*size)], RenderSettings(tile=tile, depth=depth))
+
+
+@pytest.mark.parametrize("sizes", [[(90, 70), (301, 17), (16, 200)], [(1400, 1100), (33, 33)]])
+def test_several_views(raster, sizes):
+    print("entry walk views", sizes, flush=True)
+    cloud = GaussianCloud.from_numpy(synthetic.make_cloud(20000, 6), "cuda:0")
+    # One view looks away from the cloud: its strips hold nothing.
+    views = [a_view(w, h, 0.9 * k) for k, (w, h) in enumerate(sizes)]
+    away = camera.Camera.looking_at((0.0, 0.0, 30.0), (0.0, 0.0, 60.0)).with_horizontal_fov(40.0)
+    both(raster, cloud, views + [camera.view_for(away, 64, 48)], RenderSettings())
+
+
+def test_readers_after_a_frame_without_pairs(raster):
+    print("entry walk readers", flush=True)
+    cloud = GaussianCloud.from_numpy(synthetic.make_cloud(5000, 7), "cuda:0")
+    views = [a_view(160, 90), a_view(160, 90, 1.0)]
+    settings = RenderSettings()
+    kept, _ = raster.render(views, cloud, settings, keep_backward=True)
+    want = raster.contribution(views, cloud, settings, kept, mode=1)
+    plain, _ = raster.render(views, cloud, settings)
+    assert torch.equal(raster.contribution(views, cloud, settings, plain, mode=1), want)
+    # The adjoint of the plain frame, with the walk another render kept.
+    dl = [torch.ones_like(t.colour) for t in plain]
+    grads = [{k: torch.zeros_like(getattr(cloud, k)) for k in ("means", "log_scales", "quats", "opacity_logits", "sh")}
+             for _ in range(2)]
+    plain, _ = raster.render(views, cloud, settings)
+    for t, k in zip(plain, kept):
+        t.final_t, t.last = k.final_t, k.last
+    raster.render_backward(views, cloud, settings, plain, dl, grads[0])
+    kept, _ = raster.render(views, cloud, settings, keep_backward=True)
+    raster.render_backward(views, cloud, settings, kept, dl, grads[1])
+    for name in grads[0]:
+        a, b = grads[0][name].double(), grads[1][name].double()
+        # The same sums in another order (float atomics).
+        assert float((a - b).norm()) <= 1e-4 * float(b.norm())
+
+
+def test_growth_and_async(raster):
+    """A frame of far more entries than the one before it bins twice: its total
+    is counted once. And the frame with no wait: its total, its image."""
+    print("entry walk growth", flush=True)
+    small = GaussianCloud.from_numpy(synthetic.make_cloud(300, 8), "cuda:0")
+    large = GaussianCloud.from_numpy(synthetic.make_cloud(40000, 9, log_scale_mean=-3.5), "cuda:0")
+    view, settings = a_view(400, 300), RenderSettings()
+    raster.render([view], small, settings)
+    grown, stats = raster.render([view], large, settings)
+    other = TileRasterizer(0)
+    kept, want = other.render([view], large, settings, keep_backward=True)
+    other.close()
+    assert stats.pairs == want.pairs
+    assert torch.equal(grown[0].colour, kept[0].colour)
+    drawn = raster.render_async([view], large, settings)
+    pairs, capacity = raster.frame_pairs()
+    assert pairs == want.pairs and pairs <= capacity
+    assert torch.equal(drawn[0].colour, kept[0].colour)
+    assert np.array_equal(raster.frame_buffers()["pair_values"].shape, [pairs])
