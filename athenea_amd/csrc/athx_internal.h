@@ -281,8 +281,9 @@ hipError_t launch_strip_pairs(const StripBins& b, hipStream_t s);
 hipError_t launch_big_list(const Footprints& fp, uint32_t slots, uint32_t* status_words, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
 size_t scan_status_words(uint32_t n);
+uint32_t scan_clear_words(uint32_t n);
 hipError_t launch_scan(const uint32_t* in, uint32_t* out, uint64_t* total, uint32_t n, uint32_t* status,
-                       hipStream_t s);
+                       hipStream_t s, bool cleared = false);
 // [start, end) of every key in 0..keys-1 among the first min(*n_dev, cap)
 // sorted keys (compared under key_mask); (0, 0) for a key that is absent.
 hipError_t launch_ranges(const uint32_t* sorted_keys, const uint64_t* n_dev, uint32_t cap, uint32_t keys,

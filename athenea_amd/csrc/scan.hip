@@ -536,7 +536,8 @@ __global__ void __launch_bounds__(kThreads) partition_scan_kernel(Policy pol, co
 }
 
 template <typename Policy>
-hipError_t run_scan(const Policy& pol, uint32_t max_n, uint64_t* total, uint32_t* status_words, hipStream_t s) {
+hipError_t run_scan(const Policy& pol, uint32_t max_n, uint64_t* total, uint32_t* status_words, hipStream_t s,
+                    bool cleared = false) {
     uint64_t* status = reinterpret_cast<uint64_t*>(status_words);
     const uint32_t parts = div_up(max_n ? max_n : 1, kTile);
     if (max_n > kLongScan) {
@@ -550,8 +551,10 @@ hipError_t run_scan(const Policy& pol, uint32_t max_n, uint64_t* total, uint32_t
         hipLaunchKernelGGL(partition_scan_kernel<Policy>, dim3(parts), dim3(kThreads), 0, s, pol, status, tops);
         return hipGetLastError();
     }
-    const uint32_t clear_blocks = div_up(parts + 1, 256) < 1024 ? div_up(parts + 1, 256) : 1024;
-    hipLaunchKernelGGL(clear_status_kernel<Policy>, dim3(clear_blocks), dim3(256), 0, s, pol, status, total);
+    if (!cleared) {
+        const uint32_t clear_blocks = div_up(parts + 1, 256) < 1024 ? div_up(parts + 1, 256) : 1024;
+        hipLaunchKernelGGL(clear_status_kernel<Policy>, dim3(clear_blocks), dim3(256), 0, s, pol, status, total);
+    }
     hipLaunchKernelGGL(scan_kernel<Policy>, dim3(parts), dim3(kThreads), 0, s, pol, total, status);
     return hipGetLastError();
 }
@@ -672,9 +675,14 @@ size_t scan_status_words(uint32_t n) {
     return 2 * (2 + parts + div_up64(parts, kSumThreads));
 }
 
+// The status words a caller clears before launch_scan(.., cleared): the
+// ticket's and a partition's each, two u32 a word; none for a long scan, which
+// writes its words whole.
+uint32_t scan_clear_words(uint32_t n) { return n > kLongScan ? 0u : 2u * (1u + div_up(n ? n : 1, kTile)); }
+
 hipError_t launch_scan(const uint32_t* in, uint32_t* out, uint64_t* total, uint32_t n, uint32_t* status_words,
-                       hipStream_t s) {
-    return run_scan(PlainScan{in, out, n}, n, total, status_words, s);
+                       hipStream_t s, bool cleared) {
+    return run_scan(PlainScan{in, out, n}, n, total, status_words, s, cleared && n != 0);
 }
 
 hipError_t launch_compact(const uint32_t* touched, const uint32_t* depth_keys, uint32_t slots, uint32_t* keys_out,

@@ -95,18 +95,25 @@ __host__ __device__ inline void pass_digit(uint32_t p, uint32_t lo_bit, uint32_t
     shift = lo_bit + p * base + (p < extra ? p : extra);
 }
 
-// The lanes of the wavefront whose digit equals this lane's: a ballot a bit.
+// The lanes of the wavefront whose digit equals this lane's: a ballot a bit,
+// and each half of the mask m & ~(ballot ^ the bit spread over the word) in
+// one three-input operation. Ranking a pass's keys is mostly this, and the
+// passes are bound by the VALU as much as by memory (downsweep_kernel, us a
+// pass, with selects and two-input operations and with these: 10 M 64-bit keys
+// 73.5 -> 68.4, 222 M strip entries 989 -> 914).
 __device__ inline uint64_t match_digit(uint32_t d, uint32_t width, bool ok) {
-    uint64_t m = __ballot(ok);
+    const uint64_t live = __builtin_amdgcn_ballot_w64(ok);
+    uint32_t lo = (uint32_t)live, hi = (uint32_t)(live >> 32);
 #pragma unroll
     for (uint32_t b = 0; b < 8; ++b) {
         if (b < width) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t on = __ballot(bit);
-            m &= bit ? on : ~on;
+            const uint32_t bit = (uint32_t)__builtin_amdgcn_sbfe((int)d, b, 1);  // 0 or ~0
+            const uint64_t on = __builtin_amdgcn_ballot_w64(bit != 0u);
+            lo = __builtin_amdgcn_bitop3_b32(lo, (uint32_t)on, bit, 0x90);
+            hi = __builtin_amdgcn_bitop3_b32(hi, (uint32_t)(on >> 32), bit, 0x90);
         }
     }
-    return m;
+    return (uint64_t)lo | (uint64_t)hi << 32;
 }
 
 // Every pass's digit counts in one read of the keys, a block's counts in LDS
@@ -437,11 +444,17 @@ __device__ inline uint32_t banded_part(const L& layout, uint32_t kP) {
 template <typename K, typename D, uint32_t kT, typename L>
 __global__ void __launch_bounds__(kT) upsweep_kernel(const K* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                      L layout, D digit, uint32_t width,
-                                                     uint32_t* __restrict__ counts) {
+                                                     uint32_t* __restrict__ counts, uint32_t* __restrict__ status,
+                                                     uint32_t status_words) {
     static_assert(kT >= kRadix && kT % 64 == 0, "a thread a digit");
     constexpr uint32_t kP = kT * kItems;
     __shared__ uint32_t s_hist[kRadix];
     const uint32_t tid = threadIdx.x;
+    // The words of the scan that follows, cleared here instead of by a launch
+    // of their own (some 4.5 us a pass).
+    for (uint32_t w = blockIdx.x * kT + tid; w < status_words; w += gridDim.x * kT) {
+        status[w] = 0;
+    }
     const uint32_t radix = 1u << width;
     Part pt;
     if (!layout.part(blockIdx.x, kP, pt)) {
@@ -645,9 +658,10 @@ hipError_t sort_impl(K* keys, uint32_t* values, const uint64_t* n_dev, uint32_t 
             const KeyDigit digit{shift, (1u << width) - 1u};
             const PlainLayout layout{n_dev, cap, rparts};
             hipLaunchKernelGGL((upsweep_kernel<K, KeyDigit, kT, PlainLayout>), dim3(rparts), dim3(kT), 0, s, kin, vin,
-                               layout, digit, width, sc.counts);
+                               layout, digit, width, sc.counts, sc.scan_status,
+                               scan_clear_words((1u << width) * rparts));
             if (hipError_t e = launch_scan(sc.counts, sc.offsets, sc.scan_total, (1u << width) * rparts,
-                                           sc.scan_status, s);
+                                           sc.scan_status, s, true);
                 e != hipSuccess) {
                 return e;
             }
@@ -734,8 +748,9 @@ hipError_t segment_passes(uint32_t* keys, uint32_t* values, const SegmentArgs& g
         const D digit{shift, (1u << width) - 1u};
         const SegLayout layout{g.part_seg, g.seg_start, g.seg_len, g.seg_part, g.seg_base, g.parts, 1u << width};
         hipLaunchKernelGGL((upsweep_kernel<uint32_t, D, kT, SegLayout>), dim3(parts), dim3(kT), 0, s, kin, vin, layout,
-                           digit, width, sc.counts);
-        if (hipError_t e = launch_scan(sc.counts, sc.offsets, sc.scan_total, (1u << width) * parts, sc.scan_status, s);
+                           digit, width, sc.counts, sc.scan_status, scan_clear_words((1u << width) * parts));
+        if (hipError_t e = launch_scan(sc.counts, sc.offsets, sc.scan_total, (1u << width) * parts, sc.scan_status, s,
+                                       true);
             e != hipSuccess) {
             return e;
         }
