@@ -911,65 +911,49 @@ __device__ inline bool band_extent(float a, float b, float ia, float ic, float d
     // at y = +-b xg / c.
     const float sC = __builtin_amdgcn_sqrtf(C);
     const float ym = sC * sa, xg = sC * sc;
-    const float ya = fmax_(y0, -ym), yb = fmin_(y1, ym);
+    const float ya = fmaxf(y0, -ym), yb = fminf(y1, ym);
     if (ya > yb) {
         return false;
     }
     // Right end r(y) = (-b y + sqrt(a C - det y^2)) / a is concave, the left
     // end convex: each is extreme at its widest point's row, clamped to the band.
-    const float yr = clamp_((-b * xg) * ic, ya, yb);
-    const float yl = clamp_((b * xg) * ic, ya, yb);
+    const float yr = __builtin_amdgcn_fmed3f((-b * xg) * ic, ya, yb);
+    const float yl = __builtin_amdgcn_fmed3f((b * xg) * ic, ya, yb);
     const float aC = a * C;
-    xb = (-b * yr + __builtin_amdgcn_sqrtf(fmax_(aC - det * yr * yr, 0.0f))) * ia;
-    xa = (-b * yl - __builtin_amdgcn_sqrtf(fmax_(aC - det * yl * yl, 0.0f))) * ia;
+    xb = (-b * yr + __builtin_amdgcn_sqrtf(fmaxf(aC - det * yr * yr, 0.0f))) * ia;
+    xa = (-b * yl - __builtin_amdgcn_sqrtf(fmaxf(aC - det * yl * yl, 0.0f))) * ia;
     return true;
 }
 
 // The strip columns c0 .. c1 whose box x-range meets [xa, xb] (relative to
-// the centre cx): bit j for column tx0 + j. A column's box is
-// [tx T + 0.5, min((tx + 1) T, W) - 0.5] in pixel centres, and both its
-// edges, rounded relative to cx, are nondecreasing in the column: the
-// columns meeting the extent run from the first whose right edge reaches xa
-// to the last whose left edge is at most xb. Each is found from its
-// estimate (within a column of it) by stepping while a neighbour still
-// qualifies.
-__device__ inline uint32_t columns_meeting(float xa, float xb, float cx, uint32_t T, uint32_t W, uint32_t tx0,
-                                          uint32_t c0, uint32_t c1) {
-    const auto lo_of = [&](int tx) { return ((float)__umul24((uint32_t)tx, T) + 0.5f) - cx; };
-    const auto hi_of = [&](int tx) {
-        const uint32_t e = __umul24((uint32_t)tx + 1u, T) < W ? __umul24((uint32_t)tx + 1u, T) : W;
-        return ((float)(e - 1u) + 0.5f) - cx;
-    };
-    const int lo = (int)c0, hi = (int)c1;
-    const float inv_t = 1.0f / (float)T;
-    // First column whose right edge reaches xa (hi + 1 when none).
-    int first = (int)ceilf(clamp_((xa + cx + 0.5f) * inv_t - 1.0f, (float)lo, (float)(hi + 1)));
-#pragma clang loop unroll(disable) interleave(disable) vectorize(disable)
-    while (first > lo && hi_of(first - 1) >= xa) {
-        --first;
-    }
-#pragma clang loop unroll(disable) interleave(disable) vectorize(disable)
-    while (first <= hi && hi_of(first) < xa) {
-        ++first;
-    }
-    // Last column whose left edge is at most xb (lo - 1 when none).
-    int last = (int)floorf(clamp_((xb + cx - 0.5f) * inv_t, (float)(lo - 1), (float)hi));
-#pragma clang loop unroll(disable) interleave(disable) vectorize(disable)
-    while (last < hi && lo_of(last + 1) <= xb) {
-        ++last;
-    }
-#pragma clang loop unroll(disable) interleave(disable) vectorize(disable)
-    while (last >= lo && lo_of(last) > xb) {
-        --last;
-    }
-    if (first > last) {
+// the centre cx), to within a margin: bit j for column tx0 + j. A column's box
+// is [tx T + 0.5, min((tx + 1) T, W) - 0.5] in pixel centres, so the columns run
+// from the first whose right edge reaches xa to the last whose left edge is at
+// most xb, both found by arithmetic (T is a power of two). The edges and the
+// sums round by a few units of 2^-24 (|cx| + W); `margin` is 2^-20 of that, to
+// be met by columns that must surely meet the extent (positive) or missed by
+// columns that surely do not (negative): a column in between is one the float
+// test decides. (Stepping to the exact columns with the edges as the float
+// test rounds them took four loops and some 95 of an entry's operations, this
+// 20.)
+__device__ inline uint32_t columns_meeting(float xa, float xb, float cx, float margin, uint32_t T, uint32_t W,
+                                          uint32_t tx0, uint32_t c0, uint32_t c1) {
+    const float inv_t = __builtin_amdgcn_rcpf((float)T);
+    const float lo = (float)c0, hi = (float)c1;
+    const float left = xa + cx, right = xb + cx;
+    const float first = __builtin_amdgcn_fmed3f(ceilf((left + (0.5f + margin)) * inv_t - 1.0f), lo, hi + 1.0f);
+    const float last = __builtin_amdgcn_fmed3f(floorf((right - (0.5f + margin)) * inv_t), lo - 1.0f, hi);
+    // The view's last column may be cut short: its right edge is W - 0.5.
+    if (first > last || (margin > 0.0f && left + margin > (float)W - 0.5f)) {
         return 0u;
     }
-    return ((1u << (uint32_t)(last - first + 1)) - 1u) << ((uint32_t)first - tx0);
+    const uint32_t f = (uint32_t)(int)first, l = (uint32_t)(int)last;
+    return ((2u << (l - f)) - 1u) << (f - tx0);
 }
 
-// An entry's strip columns c0 .. c1 (tile row with band terms Y): the
-// columns surely touched, and those the float test must decide.
+// An entry's strip columns c0 .. c1 (its tile row's first and last pixel
+// centres ylo, yhi relative to the centre): the columns surely touched, and
+// those the float test must decide.
 struct Decided {
     uint32_t sure, test;
 };
@@ -996,7 +980,7 @@ __device__ inline SliceTerms slice_terms(float a, float b, float c) {
     return t;
 }
 
-__device__ inline Decided decide_columns(const BigFootprint& g, const SliceTerms& S, const BoxAxis& Y, uint32_t T,
+__device__ inline Decided decide_columns(const BigFootprint& g, const SliceTerms& S, float ylo, float yhi, uint32_t T,
                                          uint32_t W, uint32_t tx0, uint32_t c0, uint32_t c1) {
     Decided d{0u, 0u};
     if (c1 < c0) {
@@ -1007,16 +991,20 @@ __device__ inline Decided decide_columns(const BigFootprint& g, const SliceTerms
         return d;
     }
     const uint32_t ex = __umul24(c1 + 1u, T) < W ? __umul24(c1 + 1u, T) : W;
-    const float X = fmax_(fabsf(((float)__umul24(c0, T) + 0.5f) - g.cx), fabsf(((float)(ex - 1u) + 0.5f) - g.cx));
-    const float Yb = fmax_(fabsf(Y.lo), fabsf(Y.hi));
+    const float X = fmaxf(fabsf(((float)__umul24(c0, T) + 0.5f) - g.cx), fabsf(((float)(ex - 1u) + 0.5f) - g.cx));
+    const float Yb = fmaxf(fabsf(ylo), fabsf(yhi));
     const float slack = kSlack * (g.a * X * X + 2.0f * fabsf(g.b) * X * Yb + g.c * Yb * Yb);
+    const float margin = 0x1p-20f * (fabsf(g.cx) + (float)W);
     float xa = 0.0f, xb = 0.0f;
-    d.sure = band_extent(g.a, g.b, g.ia, g.ic, S.det, S.sa, S.sc, g.cutoff - slack, Y.lo, Y.hi, xa, xb)
-                 ? columns_meeting(xa, xb, g.cx, T, W, tx0, c0, c1)
+    d.sure = band_extent(g.a, g.b, g.ia, g.ic, S.det, S.sa, S.sc, g.cutoff - slack, ylo, yhi, xa, xb)
+                 ? columns_meeting(xa, xb, g.cx, margin, T, W, tx0, c0, c1)
                  : 0u;
-    const uint32_t maybe = band_extent(g.a, g.b, g.ia, g.ic, S.det, S.sa, S.sc, g.cutoff + slack, Y.lo, Y.hi, xa, xb)
-                               ? columns_meeting(xa, xb, g.cx, T, W, tx0, c0, c1)
-                               : 0u;
+    uint32_t maybe = 0u;
+    if (band_extent(g.a, g.b, g.ia, g.ic, S.det, S.sa, S.sc, g.cutoff + slack, ylo, yhi, xa, xb)) {
+        // (An extent that is not one -- a NaN -- leaves every column to the test.)
+        maybe = xa <= xb ? columns_meeting(xa, xb, g.cx, -margin, T, W, tx0, c0, c1)
+                         : ((2u << (c1 - c0)) - 1u) << (c0 - tx0);
+    }
     d.test = maybe & ~d.sure;
     return d;
 }
@@ -1211,14 +1199,20 @@ __global__ void __launch_bounds__(kEmitThreads) strip_mask_emit_kernel(const DVi
         g.ia = geo2.z;
         g.ic = geo2.w;
         const uint32_t wh = __builtin_bit_cast(uint32_t, sl.w), width = wh & 0xFFFFu, height = wh >> 16;
-        const float b2 = 2.0f * g.b;
-        const BoxAxis Y = box_axis(y0 + row, T, height, g.cy, g.a, g.b, g.c, b2);
-        const Decided d = decide_columns(g, SliceTerms{sl.x, sl.y, sl.z}, Y, T, width, tx0, c0, c1);
+        const uint32_t ty = y0 + row;
+        const uint32_t ey = __umul24(ty + 1u, T) < height ? __umul24(ty + 1u, T) : height;
+        const float ylo = ((float)__umul24(ty, T) + 0.5f) - g.cy, yhi = ((float)(ey - 1u) + 0.5f) - g.cy;
+        const Decided d = decide_columns(g, SliceTerms{sl.x, sl.y, sl.z}, ylo, yhi, T, width, tx0, c0, c1);
         uint32_t mask = d.sure;
-        for (uint32_t t = d.test; t != 0; t &= t - 1u) {
-            const uint32_t bit = (uint32_t)__builtin_ctz(t);
-            if (box_hit(g, b2, box_axis(tx0 + bit, T, width, g.cx, g.c, g.b, g.a, b2), Y)) {
-                mask |= 1u << bit;
+        if (d.test != 0u) {
+            // The row's terms of the float test (two divides) only where one is left.
+            const float b2 = 2.0f * g.b;
+            const BoxAxis Y = box_axis(ty, T, height, g.cy, g.a, g.b, g.c, b2);
+            for (uint32_t t = d.test; t != 0; t &= t - 1u) {
+                const uint32_t bit = (uint32_t)__builtin_ctz(t);
+                if (box_hit(g, b2, box_axis(tx0 + bit, T, width, g.cx, g.c, g.b, g.a, b2), Y)) {
+                    mask |= 1u << bit;
+                }
             }
         }
         const uint64_t at = (uint64_t)base + gi;
@@ -1495,7 +1489,7 @@ __global__ void __launch_bounds__(kSegThreads) strip_count_kernel(StripBins b) {
             s_entry[threadIdx.x].row = make_float4(Y.lo, Y.hi, Y.q_lo, Y.q_hi);
             s_entry[threadIdx.x].more = make_float4(Y.s_lo, Y.s_hi, g.ic, g.cutoff);
             // Sure hits and sure misses from the slice's extent; the rest tested.
-            const Decided d = decide_columns(g, slice_terms(g.a, g.b, g.c), Y, T, V.width, tx0, c0, c1);
+            const Decided d = decide_columns(g, slice_terms(g.a, g.b, g.c), Y.lo, Y.hi, T, V.width, tx0, c0, c1);
             sure = d.sure;
             test = d.test;
         }
