@@ -25,7 +25,7 @@ JSON line:
   sort          athx_sort_pairs on 10M pairs with 32-bit keys (the
                 reference's own sort benchmark size): keys/s
   stages_ms     per-stage times from HIP events on the rasterizer's stream
-  roofline      the dominant kernel (blend_kernel): its VALU issue rate
+  roofline      the dominant kernel (blend_entries_kernel): its VALU issue rate
                 against MI355X's one wave instruction a CU a clock, from the
                 committed rocprofv3 counters over its live event time; its
                 HBM traffic beside it
@@ -64,7 +64,7 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def stage_bytes(n: int, visible: int, pairs: int, entries: int, tiles: int, pixels: int, relit: bool = False) -> dict:
+def stage_bytes(n: int, visible: int, entries: int, tiles: int, pixels: int, relit: bool = False) -> dict:
     """Compulsory HBM bytes per stage of one frame -- what each stage must
     read and write whatever its implementation (the per-unit figures of the
     rasterizer's algorithmic byte model: parameters and records once, (key,
@@ -80,11 +80,12 @@ def stage_bytes(n: int, visible: int, pairs: int, entries: int, tiles: int, pixe
         # the sorted slot and the record's 32 B of geometry read a drawn
         # footprint; (strip | tile mask, slot) written an entry
         "emit": visible * (4 + 32) + entries * 8,
-        # the entries read once; each pair's slot written
-        "tile_sort": entries * 8 + pairs * 4,
-        "ranges": tiles * 8,
-        # each pair's slot and record read, the targets written
-        "blend": pairs * (4 + 48) + pixels * 28,
+        # no pairs are listed: each strip's two bounds written
+        "tile_sort": 0,
+        "ranges": tiles // 16 * 8,
+        # each entry's tile mask and slot and each drawn record read once,
+        # colour and depth written
+        "blend": entries * 8 + visible * 48 + pixels * 20,
     }
 
 
@@ -304,7 +305,7 @@ def main() -> int:
     info = raster.frame_info()
 
     # Per-stage times from HIP events recorded on the rasterizer's stream:
-    # "blend" is blend_kernel's launch alone.
+    # "blend" is blend_entries_kernel's launch alone.
     staged = RenderSettings(tile=args.tile, batch=args.batch, time_stages=True, count_splats=True)
     stage_samples = {k: [] for k in STAGES}
     for _ in range(max(3, min(args.steps, 10))):
@@ -332,13 +333,13 @@ def main() -> int:
     torch.cuda.synchronize()
 
     tiles = info["tiles"]
-    sbytes = stage_bytes(cloud.count, counters.visible, pairs, info["entries"], tiles, W * H, relit=True)
+    sbytes = stage_bytes(cloud.count, counters.visible, info["entries"], tiles, W * H, relit=True)
     prof = committed_counters().get("kernels", {})
-    blend_prof = prof.get("blend_kernel", {})
+    blend_prof = prof.get("blend_entries_kernel", {})
     blend_s = stages["blend"] * 1e-3
     valu = blend_prof.get("SQ_INSTS_VALU")
     roofline = {
-        "kernel": "blend_kernel",
+        "kernel": "blend_entries_kernel",
         "bound": "valu",
         "achieved": round(valu / blend_s / 1e9, 1) if valu else None,
         "peak": round(VALU_PEAK / 1e9, 1),
@@ -394,9 +395,9 @@ def main() -> int:
         "strip_entries": info["entries"],
         "visible": counters.visible,
         "stages_ms": {k: round(v, 4) for k, v in stages.items()},
-        "stage_hbm_frac": {k: round(sbytes[k] / (stages[k] * 1e-3) / HBM_PEAK, 4) for k in STAGES if stages[k] > 0},
+        "stage_hbm_frac": {k: round(sbytes[k] / (stages[k] * 1e-3) / HBM_PEAK, 4) for k in STAGES if stages[k] > 0 and sbytes[k]},
         "depth_sort_keys_per_s": round(counters.visible / (stages["depth_sort"] * 1e-3)),
-        "pairs_binned_per_s": round(pairs / ((stages["emit"] + stages["tile_sort"]) * 1e-3)),
+        "entries_sorted_per_s": round(info["entries"] / (stages["emit"] * 1e-3)),
         "roofline": roofline,
         "roofline_hbm": roofline_hbm,
     }

@@ -412,7 +412,9 @@ ATHX_API athx_status athx_render_instances(athx_ctx* ctx, const athx_view* views
  * waits for the host. A frame with more pairs (or entries) than that room
  * draws incompletely (the reference's emit drops pairs past its capacity the
  * same way, shaders/athenea/splat/splat_emit.slang:43-46): athx_frame_pairs
- * says so.
+ * says so. A frame that lists no pairs while it draws (no targets[].last, no
+ * variants, tiles of 16 or 32) is complete once its entries fit; the pair
+ * room then bounds what a later reader of its pairs gets.
  */
 ATHX_API athx_status athx_render_async(athx_ctx* ctx, const athx_view* views, uint32_t nviews,
                                        const athx_gaussians* gaussians, const athx_settings* settings,
