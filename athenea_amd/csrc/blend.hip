@@ -1271,14 +1271,17 @@ __global__ void __launch_bounds__(TILE * TILE) blend_backward_kernel(
             br = __builtin_fmaf(alpha, or_, br);
             bgc = __builtin_fmaf(alpha, og, bgc);
             bb = __builtin_fmaf(alpha, ob, bb);
+            // (Zeroed by selection: an infinite or NaN dL/dC of a pixel reaches
+            // the Gaussians that the pixel took and no others of its block.)
             const float w = alpha * T;
-            const float u = dl_dalpha * (took & !(raw > 0.99f) ? e : 0.0f);
+            const float u = took & !(raw > 0.99f) ? dl_dalpha * e : 0.0f;
+            const float wr = took ? w * gr : 0.0f, wg = took ? w * gg : 0.0f, wb = took ? w * gb : 0.0f;
             const float ux = u * dx, uy = u * dy;
             // -2 x's derivatives along dx and dy, where a thin Gaussian's
             // terms cancel: taken a pixel, not from the pixels' sums.
             const float hx = __builtin_fmaf(-ka.w, dy, -2.0f * (ka.z * dx));
             const float hy = __builtin_fmaf(-ka.w, dx, -2.0f * (kb.x * dy));
-            const float sums[9] = {u, u * hx, ux * dx, ux * dy, u * hy, uy * dy, w * gr, w * gg, w * gb};
+            const float sums[9] = {u, u * hx, ux * dx, ux * dy, u * hy, uy * dy, wr, wg, wb};
             float s0, s1, s2;
             row_sum9(sums, s0, s1, s2);
             if (writes) {
