@@ -8,6 +8,8 @@ one: means, log-scales, quaternions, opacity logits and SH coefficients.
 """
 from __future__ import annotations
 
+import dataclasses
+
 import torch
 
 from .raster import GaussianCloud, RenderSettings, TileRasterizer
@@ -23,7 +25,9 @@ class _Rasterize(torch.autograd.Function):
         ctx.views = views
         ctx.settings = settings
         ctx.cloud = cloud
-        ctx.targets = targets
+        # The images are this node's outputs, and an output holds its node: kept
+        # here as they are, each frame would wait for the garbage collector.
+        ctx.targets = [dataclasses.replace(t, colour=t.colour.detach(), depth=t.depth.detach()) for t in targets]
         ctx.sh_dtype = sh.dtype
         for t in targets:
             ctx.mark_non_differentiable(t.depth)
