@@ -18,6 +18,7 @@
 // gradient is summed across the row first, then over the tile's rows in LDS,
 // and added to memory once a tile.
 #include "athx_internal.h"
+#include "bounds.h"
 
 namespace athx {
 namespace {
@@ -1239,11 +1240,10 @@ __global__ void __launch_bounds__(TILE * TILE) blend_backward_kernel(
         rec_now = fetch(records, slot_ahead);
         slot_ahead = pair_slots[pair_of(lo > batch ? lo - batch : 0u)];
         // Back to front over the row's Gaussians below its furthest pair.
-        const uint32_t top = row_last > lo ? (row_last - lo < count ? row_last - lo : count) : 0u;
-        const uint32_t length = expand_list(s, block, lane, top);
+        const uint32_t length = expand_list(s, block, lane, bytes_below(row_last, lo, count, 1u));
         wave_lds_fence();
         const uint16_t* list = s.list[block];
-        const uint32_t last_at = last > lo ? (last - lo) * (uint32_t)sizeof(LdsRecord) : 0u;
+        const uint32_t last_at = bytes_below(last, lo, count, (uint32_t)sizeof(LdsRecord));
         for (uint32_t i = length; i-- != 0;) {
             const uint32_t at = list[i];
             const LdsRecord& k = *reinterpret_cast<const LdsRecord*>(reinterpret_cast<const char*>(s.rec) + at);
