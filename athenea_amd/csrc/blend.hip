@@ -1177,6 +1177,8 @@ __global__ void __launch_bounds__(TILE * TILE) blend_backward_kernel(
         const float4 gc = reinterpret_cast<const float4*>(V.dl_dcolour)[pix];
         gr = gc.x; gg = gc.y; gb = gc.z; ga = gc.w;
     }
+    // A pixel of the wavefront's has a dL/dC that is not finite.
+    const bool infinite = __ballot(!(fabsf(gr) + fabsf(gg) + fabsf(gb) < INFINITY)) != 0;
     // dL/dC . (the colour of everything behind the current Gaussian, as seen
     // from just in front of it): the background, then each Gaussian over it.
     float br = V.bg[0], bgc = V.bg[1], bb = V.bg[2];
@@ -1271,11 +1273,19 @@ __global__ void __launch_bounds__(TILE * TILE) blend_backward_kernel(
             br = __builtin_fmaf(alpha, or_, br);
             bgc = __builtin_fmaf(alpha, og, bgc);
             bb = __builtin_fmaf(alpha, ob, bb);
-            // (Zeroed by selection: an infinite or NaN dL/dC of a pixel reaches
-            // the Gaussians that the pixel took and no others of its block.)
+            // Zeroed by selection: an infinite or NaN dL/dC of a pixel reaches
+            // the Gaussians that the pixel took and no others of its block.
             const float w = alpha * T;
             const float u = took & !(raw > 0.99f) ? dl_dalpha * e : 0.0f;
-            const float wr = took ? w * gr : 0.0f, wg = took ? w * gg : 0.0f, wb = took ? w * gb : 0.0f;
+            float wr = w * gr, wg = w * gg, wb = w * gb;
+            if (infinite) {
+                // (Kept a branch: the three selects in every step are 3 % of
+                // the walk, 513 us against 501 at 1920 x 1080.)
+                asm volatile("" : "+v"(wr), "+v"(wg), "+v"(wb));
+                wr = took ? wr : 0.0f;
+                wg = took ? wg : 0.0f;
+                wb = took ? wb : 0.0f;
+            }
             const float ux = u * dx, uy = u * dy;
             // -2 x's derivatives along dx and dy, where a thin Gaussian's
             // terms cancel: taken a pixel, not from the pixels' sums.
