@@ -10,6 +10,7 @@
 // depth keys, tile counts and records are the same bits a host restatement
 // computes.
 #include "athx_internal.h"
+#include "bounds.h"
 #include "relight.h"
 
 namespace athx {
@@ -850,25 +851,12 @@ __global__ void __launch_bounds__(kSettleThreads) settle_count_kernel(const DVie
             const BigFootprint g = big_footprint(views, n, T, records, slot);
             const DView& V = views[g.view];
             const uint32_t area = g.w * g.h;
-            // A long thin footprint's rectangle holds thousands of tiles that
-            // its sliver never comes near, and one wavefront walks them all: a
-            // step is left out when no tile of it reaches within the sliver's
-            // half width of its axis. q >= l (u . p)^2 with l the conic's
-            // larger eigenvalue and u its unit direction; a tile's |u . p| is
-            // at least its centre's less what its half sides span. (1 % and a
-            // hundredth of a pixel, above any rounding here, stay on the safe
-            // side; a NaN leaves nothing out. 1920x1080, 1.4 M Gaussians: 42.9 us
-            // a launch with every tile tested, 14.7 this way; where footprints
-            // are round it costs what it saves: 960x540 x 60 views, 2.36 M: 213 and 217.)
-            const float mean = 0.5f * (g.a + g.c), half = 0.5f * (g.a - g.c);
-            const float root = __builtin_amdgcn_sqrtf(half * half + g.b * g.b), larger = mean + root;
-            const float vx = half >= 0.0f ? half + root : g.b, vy = half >= 0.0f ? g.b : root - half;
-            const float norm = __builtin_amdgcn_rsqf(fmaxf(vx * vx + vy * vy, 1e-30f));
-            const float ux = vx * norm, uy = vy * norm;
-            const float side = 0.5f * (float)T;
-            const float reach = __builtin_amdgcn_sqrtf(1.01f * g.cutoff * __builtin_amdgcn_rcpf(larger)) +
-                                side * (fabsf(ux) + fabsf(uy)) + 0.01f +
-                                1e-5f * (fabsf(g.cx) + fabsf(g.cy) + (float)(V.width + V.height));
+            // A step none of whose tiles reaches the sliver (axis_reach) is
+            // left out. (1920x1080, 1.4 M Gaussians: 42.9 us a launch with every
+            // tile tested, 17.2 this way; where footprints are round it costs
+            // more than it saves: 960x540 x 60 views, 2.36 M: 213 and 223.)
+            const AxisReach axis = axis_reach(g.a, g.b, g.c, g.cutoff, g.cx, g.cy, T, V.width, V.height, g.x0, g.y0,
+                                              g.w, g.h);
             // Tile k of the rectangle, row-major: 64 on is `over` rows and
             // `on` columns on.
             const uint32_t wide = max(g.w, 1u), over = 64u / wide, on = 64u - over * wide;
@@ -876,9 +864,7 @@ __global__ void __launch_bounds__(kSettleThreads) settle_count_kernel(const DVie
             bool any = false;
             for (uint32_t k0 = 0; k0 < area && !any; k0 += 64) {
                 const uint32_t tx = g.x0 + col, ty = g.y0 + row;
-                const float px = ((float)__umul24(tx, T) + side) - g.cx, py = ((float)__umul24(ty, T) + side) - g.cy;
-                const bool apart = fabsf(ux * px + uy * py) > reach;
-                const bool near = k0 + lane < area && !apart;
+                const bool near = k0 + lane < area && !apart(axis, g.cx, g.cy, T, tx, ty);
                 if (__ballot(near) != 0) {
                     const bool hit = near && tile_touched(V.width, V.height, T, g.cx, g.cy, g.a, g.b, g.c, g.cutoff,
                                                           tx, ty);
@@ -929,8 +915,7 @@ __global__ void __launch_bounds__(kSettleThreads) settle_count_kernel(const DVie
 // same order in power (where its square root is ill-conditioned, at the
 // ellipse's top and bottom, the power's x-gradient vanishes), and the
 // determinant is taken in FP64, where a thin ellipse's does not cancel;
-// kSlack = 256 * 2^-24 covers both with a wide margin.
-constexpr float kSlack = 256.0f * 0x1p-24f;
+// kSlack (bounds.h) covers both with a wide margin.
 
 // [xa, xb]: the x-extent of {(x, y) : y0 <= y <= y1, q(x, y) <= C}
 // (coordinates relative to the centre; sa = sqrt(a / det), sc = sqrt(c /
