@@ -1183,7 +1183,9 @@ void finish_frame(athx_ctx* ctx, const athx_settings* settings, const FrameShape
 
 // The last frame's pairs and ranges for their readers (the adjoint, the
 // contributions, copy_frame), where the frame listed none: from the sorted
-// entries it left, up to its capacity as the frame itself would have.
+// entries and the views it left, up to its capacity as the frame itself would
+// have. The device's views must still be the frame's: a reader lists before it
+// uploads its own, which may be laid out otherwise.
 athx_status list_pairs(athx_ctx* ctx, hipStream_t s) {
     if (ctx->pairs_listed) {
         return ATHX_OK;
@@ -1693,10 +1695,11 @@ ATHX_API athx_status athx_render_backward(athx_ctx* ctx, const athx_view* views,
     if (tiles64 != ctx->last_tiles) {
         return fail(ctx, ATHX_INVALID_ARGUMENT, "the views differ from the rendered frame's");
     }
-    if (athx_status st = upload_views(ctx, nviews, s); st != ATHX_OK) {
+    // From the frame's own views, which the reader's then replace.
+    if (athx_status st = list_pairs(ctx, s); st != ATHX_OK) {
         return st;
     }
-    if (athx_status st = list_pairs(ctx, s); st != ATHX_OK) {
+    if (athx_status st = upload_views(ctx, nviews, s); st != ATHX_OK) {
         return st;
     }
     const uint32_t slots = gaussians->count * nviews;
@@ -1752,10 +1755,11 @@ ATHX_API athx_status athx_contribution(athx_ctx* ctx, const athx_view* views, ui
     if (tiles64 != ctx->last_tiles) {
         return fail(ctx, ATHX_INVALID_ARGUMENT, "the views differ from the rendered frame's");
     }
-    if (athx_status st = upload_views(ctx, nviews, s); st != ATHX_OK) {
+    // From the frame's own views, which the reader's then replace.
+    if (athx_status st = list_pairs(ctx, s); st != ATHX_OK) {
         return st;
     }
-    if (athx_status st = list_pairs(ctx, s); st != ATHX_OK) {
+    if (athx_status st = upload_views(ctx, nviews, s); st != ATHX_OK) {
         return st;
     }
     const uint64_t words = (uint64_t)ctx->last_n * nviews * (mode == 4 ? 4u : mode == 1 ? 1u : 2u);

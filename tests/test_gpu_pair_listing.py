@@ -1,0 +1,67 @@
+"""The pairs of a frame that listed none while it drew, listed for the first of
+their readers: the frame's own, whoever reads them, in what order and on which
+stream."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from athenea_amd import RenderSettings, TileRasterizer, _lib, synthetic
+from athenea_amd.raster import GaussianCloud, RenderTargets
+from tests.test_gpu_entry_walk import a_view
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def raster():
+    r = TileRasterizer(0)
+    yield r
+    r.close()
+
+
+@pytest.fixture(scope="module")
+def cloud():
+    return GaussianCloud.from_numpy(synthetic.make_cloud(5000, 7), "cuda:0")
+
+
+def the_pairs(raster):
+    """The last frame's pairs and ranges alone (athx_copy_frame), on the current stream."""
+    info = raster.frame_info()
+    shapes = {"pair_keys": ((info["pairs"],), torch.int64), "pair_values": ((info["pairs"],), torch.int32),
+              "ranges": ((info["tiles"], 2), torch.int32)}
+    out = {}
+    for part, (shape, dtype) in shapes.items():
+        t = out[part] = torch.zeros(shape, dtype=dtype, device="cuda:0")
+        raster._check(raster._lib.athx_copy_frame(raster._ctx, _lib.FRAME_PARTS[part], t.data_ptr(),
+                                                  t.numel() * t.element_size(), torch.cuda.current_stream().cuda_stream))
+    return out
+
+
+def listed_by_the_frame(raster, views, cloud, settings):
+    """The frame's pairs as a frame that keeps its walk lists them."""
+    raster.render(views, cloud, settings, keep_backward=True)
+    return the_pairs(raster)
+
+
+def check_pairs(got, want):
+    torch.cuda.synchronize()
+    for part in want:
+        assert torch.equal(got[part], want[part]), part
+
+
+@pytest.mark.parametrize("sizes,others", [([(160, 48), (48, 160)], [(48, 160), (160, 48)]), ([(336, 16)], [(16, 336)]),
+                                          ([(16, 336)], [(336, 16)])])
+def test_a_readers_views_do_not_lay_out_the_pairs(raster, cloud, sizes, others):
+    """A reader whose views have as many tiles as the frame's, but of another
+    shape, is taken as before; the pairs are listed from the frame's views."""
+    print("pair listing, other views", sizes, others, flush=True)
+    settings = RenderSettings()
+    views = [a_view(w, h) for w, h in sizes]
+    want = listed_by_the_frame(raster, views, cloud, settings)
+    targets, stats = raster.render(views, cloud, settings)
+    reshaped = [RenderTargets.allocate(w, h, "cuda:0", False) for w, h in others]
+    for t in reshaped:
+        t.frame_serial = stats.frame_serial
+    raster.contribution([a_view(w, h) for w, h in others], cloud, settings, reshaped, mode=1)
+    check_pairs(the_pairs(raster), want)
