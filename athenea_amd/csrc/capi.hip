@@ -149,6 +149,11 @@ struct athx_ctx {
     bool last_strips_in_alt = false;  // the sorted strip entries are in the strip_alt buffers
     FrameShape last_shape;            // the sizes the last frame ran at
     bool pairs_listed = true;         // its pairs and ranges are in pair_vals and ranges (list_pairs)
+    // A listing queued on a reader's stream: other streams' readers, and the
+    // next frame, wait for it (wait_listed).
+    hipEvent_t listed_done = nullptr;
+    hipStream_t listed_stream = nullptr;
+    bool listing = false;
     // The last frame sorted each view's slots apart (its ranks grouped by
     // view): the exact offsets, scanned in the frame's whole depth order,
     // then sort that order on request (order_* buffers).
@@ -1177,8 +1182,27 @@ void finish_frame(athx_ctx* ctx, const athx_settings* settings, const FrameShape
     ctx->last_true_pairs = pairs_known;
     ctx->last_shape = fs;
     ctx->pairs_listed = !fs.direct;
+    ctx->listing = false;  // the frame came after it
     ctx->have_frame = true;
     ctx->serial += 1;
+}
+
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &status) == hipSuccess && status == hipStreamCaptureStatusActive;
+}
+
+// What stream s queues from here on comes after a listing that another stream
+// queued (list_pairs). A capture cannot wait for work outside it: the host does.
+athx_status wait_listed(athx_ctx* ctx, hipStream_t s) {
+    if (ctx->listing && s != ctx->listed_stream) {
+        if (capturing(s)) {
+            ATHX_HIP(ctx, hipEventSynchronize(ctx->listed_done), "wait for the listing");
+        } else {
+            ATHX_HIP(ctx, hipStreamWaitEvent(s, ctx->listed_done, 0), "wait for the listing");
+        }
+    }
+    return ATHX_OK;
 }
 
 // The last frame's pairs and ranges for their readers (the adjoint, the
@@ -1186,9 +1210,13 @@ void finish_frame(athx_ctx* ctx, const athx_settings* settings, const FrameShape
 // entries and the views it left, up to its capacity as the frame itself would
 // have. The device's views must still be the frame's: a reader lists before it
 // uploads its own, which may be laid out otherwise.
+//
+// The listing is queued on the first reader's stream; a reader on another
+// waits for it there. A reader that is being captured lists for itself: what
+// it queues runs at the replays and marks nothing listed now.
 athx_status list_pairs(athx_ctx* ctx, hipStream_t s) {
     if (ctx->pairs_listed) {
-        return ATHX_OK;
+        return wait_listed(ctx, s);
     }
     FrameShape fs = ctx->last_shape;
     fs.direct = false;
@@ -1203,7 +1231,12 @@ athx_status list_pairs(athx_ctx* ctx, hipStream_t s) {
     ATHX_HIP(ctx, launch_strip_pairs(b, s), "pairs");
     ATHX_HIP(ctx, launch_tile_ranges(b, as<uint32_t>(ctx->tile_bases), fs.tiles, as<uint32_t>(ctx->ranges), s),
              "ranges");
-    ctx->pairs_listed = true;
+    if (!capturing(s)) {
+        ATHX_HIP(ctx, hipEventRecord(ctx->listed_done, s), "record the listing");
+        ctx->listed_stream = s;
+        ctx->listing = true;
+        ctx->pairs_listed = true;
+    }
     return ATHX_OK;
 }
 
@@ -1269,6 +1302,7 @@ ATHX_API athx_status athx_create(int device, athx_ctx** out) {
         }
     }
     if (hipEventCreateWithFlags(&ctx->upload_done, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&ctx->listed_done, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&ctx->async_done, hipEventDisableTiming) != hipSuccess) {
         athx_destroy(ctx);
         return ATHX_DEVICE_FAILURE;
@@ -1335,6 +1369,9 @@ ATHX_API void athx_destroy(athx_ctx* ctx) {
     if (ctx->async_done) {
         (void)hipEventDestroy(ctx->async_done);
     }
+    if (ctx->listed_done) {
+        (void)hipEventDestroy(ctx->listed_done);
+    }
     delete ctx;
 }
 
@@ -1392,6 +1429,9 @@ athx_status render_frame(athx_ctx* ctx, const athx_view* views, uint32_t nviews,
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool timed = settings->time_stages != 0 && ctx->ev[7] != nullptr;
     const auto wall0 = std::chrono::steady_clock::now();
+    if (athx_status st = wait_listed(ctx, s); st != ATHX_OK) {
+        return st;
+    }
     if (athx_status st = upload_views(ctx, nviews, s, ninst); st != ATHX_OK) {
         return st;
     }
@@ -1582,6 +1622,9 @@ ATHX_API athx_status athx_render_async(athx_ctx* ctx, const athx_view* views, ui
     fs.capacity = (uint32_t)cap;
     set_entry_cap(fs, (uint32_t)entry_cap);
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (athx_status st = wait_listed(ctx, s); st != ATHX_OK) {
+        return st;
+    }
     if (athx_status st = upload_views(ctx, nviews, s); st != ATHX_OK) {
         return st;
     }

@@ -20,9 +20,14 @@ def raster():
     r.close()
 
 
+OTHER = []
+
+
 @pytest.fixture(scope="module")
 def cloud():
-    return GaussianCloud.from_numpy(synthetic.make_cloud(5000, 7), "cuda:0")
+    OTHER[:] = [GaussianCloud.from_numpy(synthetic.make_cloud(4000, 8), "cuda:0")]
+    yield GaussianCloud.from_numpy(synthetic.make_cloud(5000, 7), "cuda:0")
+    OTHER.clear()
 
 
 def the_pairs(raster):
@@ -39,14 +44,18 @@ def the_pairs(raster):
 
 
 def listed_by_the_frame(raster, views, cloud, settings):
-    """The frame's pairs as a frame that keeps its walk lists them."""
+    """The frame's pairs as a frame that keeps its walk lists them; the pairs of
+    another cloud are left in the buffers."""
     raster.render(views, cloud, settings, keep_backward=True)
-    return the_pairs(raster)
+    want = the_pairs(raster)
+    raster.render(views, OTHER[0], settings, keep_backward=True)
+    assert not torch.equal(the_pairs(raster)["ranges"], want["ranges"])
+    return want
 
 
 def check_pairs(got, want):
     torch.cuda.synchronize()
-    for part in want:
+    for part in got:
         assert torch.equal(got[part], want[part]), part
 
 
@@ -65,3 +74,61 @@ def test_a_readers_views_do_not_lay_out_the_pairs(raster, cloud, sizes, others):
         t.frame_serial = stats.frame_serial
     raster.contribution([a_view(w, h) for w, h in others], cloud, settings, reshaped, mode=1)
     check_pairs(the_pairs(raster), want)
+
+
+def late(stream, cycles=100_000_000):
+    """Some tens of milliseconds of work on the stream."""
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(cycles)
+
+
+def test_readers_and_frames_on_other_streams(raster, cloud):
+    """The first reader's stream is busy: its listing runs late. A reader and
+    a frame on other streams come after it."""
+    print("pair listing, streams", flush=True)
+    settings, views = RenderSettings(), [a_view(160, 90), a_view(97, 130, 1.0)]
+    want = listed_by_the_frame(raster, views, cloud, settings)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    image = raster.render(views, cloud, settings)[0][1].colour.clone()
+    torch.cuda.synchronize()
+
+    late(first)
+    with torch.cuda.stream(first):
+        early = the_pairs(raster)
+    with torch.cuda.stream(second):
+        got = the_pairs(raster)
+    check_pairs(got, want)
+    check_pairs(early, want)
+
+    raster.render(views, cloud, settings)
+    late(first)
+    with torch.cuda.stream(first):
+        early = the_pairs(raster)
+    del early["pair_keys"]  # (read from the depth keys, which the next frame replaces)
+    with torch.cuda.stream(second):
+        targets, _ = raster.render(views, cloud, settings)
+        got = the_pairs(raster)
+    check_pairs(got, want)
+    check_pairs(early, want)
+    assert torch.equal(targets[1].colour, image)
+
+
+def test_a_captured_reader(raster, cloud):
+    """A reader recorded into a graph lists at each replay, and leaves the
+    listing to do for who reads before the first."""
+    print("pair listing, captured", flush=True)
+    settings, views = RenderSettings(), [a_view(160, 90)]
+    want = listed_by_the_frame(raster, views, cloud, settings)
+    raster.render(views, cloud, settings)
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        captured = the_pairs(raster)
+    check_pairs(the_pairs(raster), want)
+    for _ in range(3):
+        for t in captured.values():
+            t.zero_()
+        graph.replay()
+        check_pairs(captured, want)
+        check_pairs(the_pairs(raster), want)
