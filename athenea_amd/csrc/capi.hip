@@ -133,7 +133,7 @@ struct athx_ctx {
     // The PLY ingest: each vertex's keep flag, their scan, the kept total.
     DeviceBuffer ingest_keep, ingest_dest, ingest_total;
     // The ground truth and the image comparisons.
-    DeviceBuffer ref_records, ref_keys, ref_values, ref_alt_keys, ref_alt_values, ref_sort_meta, ref_count;
+    DeviceBuffer ref_views, ref_records, ref_keys, ref_values, ref_alt_keys, ref_alt_values, ref_sort_meta, ref_count;
     DeviceBuffer cmp_rows, cmp_row_error, cmp_bins;
     uint64_t* host_totals = nullptr;  // pinned: the totals words (kTotal*)
     DView* host_views = nullptr;      // pinned staging for the views
@@ -206,7 +206,7 @@ std::vector<DeviceBuffer*> all_buffers(athx_ctx* ctx) {
             &ctx->strip_ranges, &ctx->segbase, &ctx->seg_map, &ctx->rank_fp, &ctx->tally, &ctx->masks, &ctx->seg_table, &ctx->exact, &ctx->exact_offsets,
             &ctx->exact_status, &ctx->api_sort_meta, &ctx->api_alt_keys, &ctx->api_alt_vals, &ctx->api_scan_status,
             &ctx->api_count, &ctx->ingest_keep, &ctx->ingest_dest, &ctx->ingest_total, &ctx->ref_records,
-            &ctx->ref_keys, &ctx->ref_values, &ctx->ref_alt_keys, &ctx->ref_alt_values, &ctx->ref_sort_meta,
+            &ctx->ref_views, &ctx->ref_keys, &ctx->ref_values, &ctx->ref_alt_keys, &ctx->ref_alt_values, &ctx->ref_sort_meta,
             &ctx->ref_count, &ctx->cmp_rows, &ctx->cmp_row_error, &ctx->cmp_bins};
 }
 
@@ -2799,9 +2799,13 @@ athx_status reference_frame(athx_ctx* ctx, const athx_view* view, const FrameIns
         return st;
     }
     const hipStream_t s = nullptr;
-    if (athx_status st = upload_views(ctx, 1, s, ninst); st != ATHX_OK) {
-        return st;
-    }
+    // Views of its own: the last frame's pairs are listed from the frame's
+    // (list_pairs), whenever their first reader comes.
+    ATHX_HIP(ctx, reserve(ctx, ctx->ref_views, sizeof(DView) * ninst), "reference views");
+    ATHX_HIP(ctx, hipMemcpyAsync(ctx->ref_views.ptr, ctx->host_views, sizeof(DView) * ninst, hipMemcpyHostToDevice, s),
+             "upload views");
+    ATHX_HIP(ctx, hipEventRecord(ctx->upload_done, s), "record upload");
+    ctx->upload_pending = true;
     const uint32_t n = (uint32_t)total;
     const size_t cap = n ? n : 1;
     ATHX_HIP(ctx, reserve(ctx, ctx->ref_records, cap * kRecordFloats * 4), "reference records");
@@ -2821,7 +2825,7 @@ athx_status reference_frame(athx_ctx* ctx, const athx_view* view, const FrameIns
         const athx_packed_splats* pk = inst[j].g->packed;
         ATHX_HIP(ctx, launch_ref_project(pk->positions, pk->shape, pk->sh, inst[j].g->count, pk->rest_per_colour,
                                          settings->max_sh_degree, settings->antialias, settings->linear,
-                                         as<DView>(ctx->views) + j, rec, as<uint32_t>(ctx->ref_keys),
+                                         as<DView>(ctx->ref_views) + j, rec, as<uint32_t>(ctx->ref_keys),
                                          as<uint32_t>(ctx->ref_values), s, base),
                  "reference projection");
         base += inst[j].g->count;
@@ -2834,7 +2838,7 @@ athx_status reference_frame(athx_ctx* ctx, const athx_view* view, const FrameIns
                               sc, s, nullptr),
              "reference sort");
     uint32_t* over = reinterpret_cast<uint32_t*>(count + 1);
-    ATHX_HIP(ctx, launch_ref_blend(as<DView>(ctx->views), view->width, view->height, rec, as<uint32_t>(ctx->ref_keys),
+    ATHX_HIP(ctx, launch_ref_blend(as<DView>(ctx->ref_views), view->width, view->height, rec, as<uint32_t>(ctx->ref_keys),
                                    as<uint32_t>(ctx->ref_values), n, 1024, settings->depth_mode,
                                    settings->depth_threshold, over, s),
              "reference blend");

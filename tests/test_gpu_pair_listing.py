@@ -8,7 +8,9 @@ import torch
 
 from athenea_amd import RenderSettings, TileRasterizer, _lib, synthetic
 from athenea_amd.raster import GaussianCloud, RenderTargets
+from athenea_amd.reference import reference_render
 from tests.test_gpu_entry_walk import a_view
+from tests.test_gpu_reference import on_device, packed_cloud
 
 pytestmark = pytest.mark.gpu
 
@@ -73,6 +75,17 @@ def test_a_readers_views_do_not_lay_out_the_pairs(raster, cloud, sizes, others):
     for t in reshaped:
         t.frame_serial = stats.frame_serial
     raster.contribution([a_view(w, h) for w, h in others], cloud, settings, reshaped, mode=1)
+    check_pairs(the_pairs(raster), want)
+
+
+def test_a_ground_truth_in_between(raster, cloud):
+    """The ground truth of another view, drawn between a frame and its reader,
+    leaves the frame's views alone."""
+    print("pair listing, ground truth", flush=True)
+    settings, views = RenderSettings(), [a_view(160, 90), a_view(97, 130, 1.0)]
+    want = listed_by_the_frame(raster, views, cloud, settings)
+    raster.render(views, cloud, settings)
+    reference_render(raster, a_view(33, 200), on_device(packed_cloud(500)), settings)
     check_pairs(the_pairs(raster), want)
 
 
