@@ -737,10 +737,9 @@ athx_status reserve_bins(athx_ctx* ctx, const FrameShape& fs) {
     return ATHX_OK;
 }
 
+// (Of a frame that lists no pairs too: its first reader then allocates nothing,
+// so that it can be captured, and where memory runs out the frame says so.)
 athx_status reserve_pairs(athx_ctx* ctx, const FrameShape& fs) {
-    if (fs.direct) {
-        return ATHX_OK;
-    }
     ATHX_HIP(ctx, reserve(ctx, ctx->pair_vals, (size_t)fs.capacity * 4 + 16), "pair values");
     return ATHX_OK;
 }
@@ -1218,11 +1217,7 @@ athx_status list_pairs(athx_ctx* ctx, hipStream_t s) {
     if (ctx->pairs_listed) {
         return wait_listed(ctx, s);
     }
-    FrameShape fs = ctx->last_shape;
-    fs.direct = false;
-    if (athx_status st = reserve_pairs(ctx, fs); st != ATHX_OK) {
-        return st;
-    }
+    const FrameShape& fs = ctx->last_shape;
     if (athx_status st = enqueue_segment_counts(ctx, fs, fs.count, ctx->last_tile, s, ctx->last_strips_in_alt);
         st != ATHX_OK) {
         return st;
@@ -1520,11 +1515,14 @@ athx_status render_frame(athx_ctx* ctx, const athx_view* views, uint32_t nviews,
     }
     const uint64_t pairs64 = host[kTotalPairs];
     if (fs.direct) {
-        // No pair buffer bounds the frame; its readers' would be this large.
+        // No pair buffer bounds the frame, only its readers.
         if (pairs64 >= kMaxPairs) {
             return fail(ctx, ATHX_UNSUPPORTED, "more than 2^30 (tile, Gaussian) pairs in one frame");
         }
-        fs.capacity = std::max<uint32_t>((uint32_t)pairs64, 1u);
+        fs.capacity = std::max<uint32_t>(std::max<uint32_t>((uint32_t)pairs64, fs.capacity), 1u);
+        if (athx_status st = reserve_pairs(ctx, fs); st != ATHX_OK) {
+            return st;
+        }
     }
     ctx->entry_last = std::min<uint64_t>(grown(host[kTotalEntries]), kMaxPairs - 1);
     ctx->pair_last = std::min<uint64_t>(grown(pairs64), kMaxPairs - 1);
@@ -2330,8 +2328,10 @@ ATHX_API athx_status athx_graph_create(int device, const athx_view* views, uint3
     if (athx_status st = reserve_bins(ctx, fs); st != ATHX_OK) {
         return graph_fail(g, st, error, error_bytes);
     }
-    if (athx_status st = reserve_pairs(ctx, fs); st != ATHX_OK) {
-        return graph_fail(g, st, error, error_bytes);
+    if (!fs.direct) {  // (a graph's frames have no readers but its own adjoint)
+        if (athx_status st = reserve_pairs(ctx, fs); st != ATHX_OK) {
+            return graph_fail(g, st, error, error_bytes);
+        }
     }
     if (settings && settings->count_splats) {
         if (athx_status st = reserve_exact(ctx, fs.slots); st != ATHX_OK) {

@@ -78,6 +78,21 @@ def test_a_readers_views_do_not_lay_out_the_pairs(raster, cloud, sizes, others):
     check_pairs(the_pairs(raster), want)
 
 
+@pytest.mark.parametrize("queued", [False, True])
+def test_the_first_reader_allocates_nothing(raster, cloud, queued):
+    print("pair listing, scratch", queued, flush=True)
+    settings, views = RenderSettings(), [a_view(160, 90), a_view(97, 130, 1.0)]
+    if queued:
+        targets = raster.render_async(views, cloud, settings, pair_capacity=200000)
+    else:
+        targets, _ = raster.render(views, cloud, settings)
+    held = raster.scratch_bytes()
+    pairs = the_pairs(raster)
+    raster.contribution(views, cloud, settings, targets, mode=1)
+    assert pairs["pair_values"].numel() > 0
+    assert raster.scratch_bytes() == held
+
+
 def test_a_ground_truth_in_between(raster, cloud):
     """The ground truth of another view, drawn between a frame and its reader,
     leaves the frame's views alone."""
