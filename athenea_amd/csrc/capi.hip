@@ -149,6 +149,9 @@ struct athx_ctx {
     bool last_strips_in_alt = false;  // the sorted strip entries are in the strip_alt buffers
     FrameShape last_shape;            // the sizes the last frame ran at
     bool pairs_listed = true;         // its pairs and ranges are in pair_vals and ranges (list_pairs)
+    // The device's views and strip entries are the last frame's: cleared when a
+    // frame begins to replace them, set when it is finished.
+    bool entries_kept = false;
     // A listing queued on a reader's stream: other streams' readers, and the
     // next frame, wait for it (wait_listed).
     hipEvent_t listed_done = nullptr;
@@ -1181,6 +1184,7 @@ void finish_frame(athx_ctx* ctx, const athx_settings* settings, const FrameShape
     ctx->last_true_pairs = pairs_known;
     ctx->last_shape = fs;
     ctx->pairs_listed = !fs.direct;
+    ctx->entries_kept = true;
     ctx->listing = false;  // the frame came after it
     ctx->have_frame = true;
     ctx->serial += 1;
@@ -1216,6 +1220,10 @@ athx_status wait_listed(athx_ctx* ctx, hipStream_t s) {
 athx_status list_pairs(athx_ctx* ctx, hipStream_t s) {
     if (ctx->pairs_listed) {
         return wait_listed(ctx, s);
+    }
+    if (!ctx->entries_kept) {
+        return fail(ctx, ATHX_INVALID_ARGUMENT,
+                    "a frame that failed has replaced the last one's entries: render it again to read its pairs");
     }
     const FrameShape& fs = ctx->last_shape;
     if (athx_status st = enqueue_segment_counts(ctx, fs, fs.count, ctx->last_tile, s, ctx->last_strips_in_alt);
@@ -1427,6 +1435,7 @@ athx_status render_frame(athx_ctx* ctx, const athx_view* views, uint32_t nviews,
     if (athx_status st = wait_listed(ctx, s); st != ATHX_OK) {
         return st;
     }
+    ctx->entries_kept = false;
     if (athx_status st = upload_views(ctx, nviews, s, ninst); st != ATHX_OK) {
         return st;
     }
@@ -1623,6 +1632,7 @@ ATHX_API athx_status athx_render_async(athx_ctx* ctx, const athx_view* views, ui
     if (athx_status st = wait_listed(ctx, s); st != ATHX_OK) {
         return st;
     }
+    ctx->entries_kept = false;
     if (athx_status st = upload_views(ctx, nviews, s); st != ATHX_OK) {
         return st;
     }

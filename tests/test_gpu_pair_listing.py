@@ -104,6 +104,30 @@ def test_a_ground_truth_in_between(raster, cloud):
     check_pairs(the_pairs(raster), want)
 
 
+def test_a_frame_that_failed_in_between(raster, cloud):
+    """A frame of more strip entries than one holds (300 000 Gaussians over
+    each of 4096 strips) is refused once it has replaced the last one's
+    entries: that one's pairs, not listed yet, are refused too."""
+    print("pair listing, failed frame", flush=True)
+    settings, views = RenderSettings(), [a_view(160, 90), a_view(97, 130, 1.0)]
+    want = listed_by_the_frame(raster, views, cloud, settings)
+    targets, _ = raster.render(views, cloud, settings)
+    crowd = synthetic.make_cloud(300000, 3)
+    crowd.log_scales[:] = 3.0
+    crowd.opacity_logits[:] = 2.0
+    with pytest.raises(_lib.AthxError) as refused:
+        raster.render([a_view(4096, 4096)], GaussianCloud.from_numpy(crowd, "cuda:0"), settings)
+    assert refused.value.code == "Unsupported"
+    with pytest.raises(_lib.AthxError) as gone:
+        the_pairs(raster)
+    assert gone.value.code == "InvalidArgument"
+    with pytest.raises(_lib.AthxError) as gone:
+        raster.contribution(views, cloud, settings, targets, mode=1)
+    assert gone.value.code == "InvalidArgument"
+    raster.render(views, cloud, settings)
+    check_pairs(the_pairs(raster), want)
+
+
 def late(stream, cycles=100_000_000):
     """Some tens of milliseconds of work on the stream."""
     with torch.cuda.stream(stream):
