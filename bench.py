@@ -18,7 +18,8 @@ JSON line:
                 (loss L2 against a target rendered from jittered means and SH)
   batched       the 60-view walk (2.36M Gaussians, 960x540 views): views/s
                 as one captured graph, with the tile side and blend batch the
-                autotuner picks, against the same views rendered one launch
+                autotuner picks (the batch is the caller's where it does not
+                reach the launch), against the same views rendered one launch
                 each
   mixed         20M Gaussians with FP16 SH, 8 views from 640x360 to 3840x2160
                 in one frame: ms/frame, views/s, pairs, strip entries

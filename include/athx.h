@@ -246,7 +246,10 @@ typedef struct athx_gaussians {
  */
 typedef struct athx_settings {
     uint32_t tile;         /* tile side in pixels: 8, 16 or 32 (the reference's is 16) */
-    uint32_t batch;        /* Gaussians staged in LDS per blend batch: 32..256, a multiple of 32 */
+    uint32_t batch;        /* Gaussians staged in LDS per batch of listed pairs: 32..256, a multiple of 32. It
+                              governs tiles of 8, frames with targets[].last or variants, frames past 65 536
+                              strips, and the contributions; other frames are blended from their strip entries,
+                              and the adjoint walks, in batches of their own. No result depends on it */
     uint32_t antialias;    /* 1: the Mip-Splatting compensation (RenderSettings::antialias) */
     uint32_t linear;       /* 1: colours are linear light; 0: sRGB, decoded per splat */
     uint32_t max_sh_degree;
