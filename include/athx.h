@@ -417,14 +417,19 @@ ATHX_API athx_status athx_render_instances(athx_ctx* ctx, const athx_view* views
  * same way, shaders/athenea/splat/splat_emit.slang:43-46): athx_frame_pairs
  * says so. A frame that lists no pairs while it draws (no targets[].last, no
  * variants, tiles of 16 or 32) is complete once its entries fit; the pair
- * room then bounds what a later reader of its pairs gets.
+ * room then bounds what a later reader of its pairs gets: with more pairs than
+ * room, the copied pairs and ranges, the contributions and the adjoint are
+ * those of the pairs that fit, under an image that holds them all.
+ * athx_frame_pairs reports more pairs than the capacity then too, as it does
+ * for a frame whose entries did not fit.
  */
 ATHX_API athx_status athx_render_async(athx_ctx* ctx, const athx_view* views, uint32_t nviews,
                                        const athx_gaussians* gaussians, const athx_settings* settings,
                                        const athx_targets* targets, uint64_t pair_capacity, void* stream);
 
 /* The last frame's pair total and its pair capacity; waits for an async
- * frame. pairs > capacity: that frame was incomplete, draw it again with
+ * frame. pairs > capacity: that frame, or what its readers get of its pairs
+ * (athx_render_async), was incomplete, draw it again with
  * a capacity of at least pairs (a frame whose strip entries outgrew their
  * room also reports more pairs than its capacity; the next frame is given
  * room for them). */

@@ -93,6 +93,32 @@ def test_the_first_reader_allocates_nothing(raster, cloud, queued):
     assert raster.scratch_bytes() == held
 
 
+@pytest.mark.parametrize("views", [1, 2])
+def test_more_pairs_than_a_queued_frame_has_room_for(raster, cloud, views):
+    """The image is whole; what is read of the pairs is their first that fit,
+    as of a frame that lists them while it draws."""
+    print("pair listing, small capacity", views, flush=True)
+    settings, views = RenderSettings(), [a_view(160, 90), a_view(97, 130, 1.0)][:views]
+    whole, stats = raster.render(views, cloud, settings)
+    want = the_pairs(raster)
+    room = stats.pairs // 3
+    kept = raster.render_async(views, cloud, settings, pair_capacity=room, keep_backward=True)
+    cut = raster.contribution(views, cloud, settings, kept, mode=1)
+    kept_pairs = the_pairs(raster)
+    targets = raster.render_async(views, cloud, settings, pair_capacity=room)
+    got = raster.contribution(views, cloud, settings, targets, mode=1)
+    assert raster.frame_pairs() == (stats.pairs, room)
+    for t, w in zip(targets, whole):
+        assert torch.equal(t.colour, w.colour) and torch.equal(t.depth, w.depth)
+    assert torch.equal(got, cut) and int(got.sum()) > 0
+    pairs = the_pairs(raster)
+    check_pairs(pairs, kept_pairs)
+    assert torch.equal(pairs["pair_values"], want["pair_values"][:room])
+    clipped = torch.clamp(want["ranges"], max=room)
+    clipped[clipped[:, 0] >= clipped[:, 1]] = 0
+    assert torch.equal(pairs["ranges"], clipped)
+
+
 def test_a_ground_truth_in_between(raster, cloud):
     """The ground truth of another view, drawn between a frame and its reader,
     leaves the frame's views alone."""
