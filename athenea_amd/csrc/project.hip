@@ -900,133 +900,6 @@ __global__ void __launch_bounds__(kSettleThreads) settle_count_kernel(const DVie
     }
 }
 
-// Deciding most of an entry's tiles without the float tile test. The test
-// (box_hit) evaluates a x^2 + 2 b x y + c y^2 at points of the tile's box
-// whose coordinates are the box edges rounded relative to the centre, in
-// about ten float operations; its result differs from the exact least power
-// over the exact box by a few units of 2^-24 M, M = a X^2 + 2 |b| X Y + c Y^2
-// with X, Y the box's largest distances from the centre. The exact least
-// power over a tile box is at most C exactly when the box's x-range meets
-// the x-extent of the ellipse q <= C sliced by the box's row band (the slice
-// is convex and spans the band's height). That extent is computed here in
-// float, once an entry, at C = cutoff -+ kSlack M: a tile meeting the inner
-// one is touched by the float test, a tile missing the outer one is not, and
-// only the tiles in between are tested. The extent's own rounding is of the
-// same order in power (where its square root is ill-conditioned, at the
-// ellipse's top and bottom, the power's x-gradient vanishes), and the
-// determinant is taken in FP64, where a thin ellipse's does not cancel;
-// kSlack (bounds.h) covers both with a wide margin.
-
-// [xa, xb]: the x-extent of {(x, y) : y0 <= y <= y1, q(x, y) <= C}
-// (coordinates relative to the centre; sa = sqrt(a / det), sc = sqrt(c /
-// det)); false when it is empty.
-__device__ inline bool band_extent(float a, float b, float ia, float ic, float det, float sa, float sc, float C,
-                                   float y0, float y1, float& xa, float& xb) {
-    if (!(C > 0.0f)) {
-        return false;
-    }
-    // The ellipse's rows: |y| <= sqrt(a C / det); its widest points (x = -+xg)
-    // at y = +-b xg / c.
-    const float sC = __builtin_amdgcn_sqrtf(C);
-    const float ym = sC * sa, xg = sC * sc;
-    const float ya = fmaxf(y0, -ym), yb = fminf(y1, ym);
-    if (ya > yb) {
-        return false;
-    }
-    // Right end r(y) = (-b y + sqrt(a C - det y^2)) / a is concave, the left
-    // end convex: each is extreme at its widest point's row, clamped to the band.
-    const float yr = __builtin_amdgcn_fmed3f((-b * xg) * ic, ya, yb);
-    const float yl = __builtin_amdgcn_fmed3f((b * xg) * ic, ya, yb);
-    const float aC = a * C;
-    xb = (-b * yr + __builtin_amdgcn_sqrtf(fmaxf(aC - det * yr * yr, 0.0f))) * ia;
-    xa = (-b * yl - __builtin_amdgcn_sqrtf(fmaxf(aC - det * yl * yl, 0.0f))) * ia;
-    return true;
-}
-
-// The strip columns c0 .. c1 whose box x-range meets [xa, xb] (relative to
-// the centre cx), to within a margin: bit j for column tx0 + j. A column's box
-// is [tx T + 0.5, min((tx + 1) T, W) - 0.5] in pixel centres, so the columns run
-// from the first whose right edge reaches xa to the last whose left edge is at
-// most xb, both found by arithmetic (T is a power of two). The edges and the
-// sums round by a few units of 2^-24 (|cx| + W); `margin` is 2^-20 of that, to
-// be met by columns that must surely meet the extent (positive) or missed by
-// columns that surely do not (negative): a column in between is one the float
-// test decides. (Stepping to the exact columns with the edges as the float
-// test rounds them took four loops and some 95 of an entry's operations, this
-// 20.)
-__device__ inline uint32_t columns_meeting(float xa, float xb, float cx, float margin, uint32_t T, uint32_t W,
-                                          uint32_t tx0, uint32_t c0, uint32_t c1) {
-    const float inv_t = __builtin_amdgcn_rcpf((float)T);
-    const float lo = (float)c0, hi = (float)c1;
-    const float left = xa + cx, right = xb + cx;
-    const float first = __builtin_amdgcn_fmed3f(ceilf((left + (0.5f + margin)) * inv_t - 1.0f), lo, hi + 1.0f);
-    const float last = __builtin_amdgcn_fmed3f(floorf((right - (0.5f + margin)) * inv_t), lo - 1.0f, hi);
-    // The view's last column may be cut short: its right edge is W - 0.5.
-    if (first > last || (margin > 0.0f && left + margin > (float)W - 0.5f)) {
-        return 0u;
-    }
-    const uint32_t f = (uint32_t)(int)first, l = (uint32_t)(int)last;
-    return ((2u << (l - f)) - 1u) << (f - tx0);
-}
-
-// An entry's strip columns c0 .. c1 (its tile row's first and last pixel
-// centres ylo, yhi relative to the centre): the columns surely touched, and
-// those the float test must decide.
-struct Decided {
-    uint32_t sure, test;
-};
-
-// A footprint's slice terms: its conic's determinant a c - b^2 (taken in
-// FP64, where a thin ellipse's does not cancel, and rounded once),
-// sqrt(a / det) and sqrt(c / det); det = 0 marks a conic the extents do
-// not handle (not positive definite, or a determinant outside the normal
-// float range), whose columns all go to the float test.
-struct SliceTerms {
-    float det, sa, sc;
-};
-
-__device__ inline SliceTerms slice_terms(float a, float b, float c) {
-    SliceTerms t{0.0f, 0.0f, 0.0f};
-    const double detd = (double)a * (double)c - (double)b * (double)b;
-    const float det = (float)detd;
-    if (a > 1e-9f && c > 1e-9f && det >= 0x1p-126f && det <= 0x1p126f) {
-        const float inv_det = __builtin_amdgcn_rcpf(det);
-        t.det = det;
-        t.sa = __builtin_amdgcn_sqrtf(a * inv_det);
-        t.sc = __builtin_amdgcn_sqrtf(c * inv_det);
-    }
-    return t;
-}
-
-__device__ inline Decided decide_columns(const BigFootprint& g, const SliceTerms& S, float ylo, float yhi, uint32_t T,
-                                         uint32_t W, uint32_t tx0, uint32_t c0, uint32_t c1) {
-    Decided d{0u, 0u};
-    if (c1 < c0) {
-        return d;
-    }
-    if (S.det == 0.0f) {
-        d.test = ((1u << (c1 - c0 + 1u)) - 1u) << (c0 - tx0);
-        return d;
-    }
-    const uint32_t ex = __umul24(c1 + 1u, T) < W ? __umul24(c1 + 1u, T) : W;
-    const float X = fmaxf(fabsf(((float)__umul24(c0, T) + 0.5f) - g.cx), fabsf(((float)(ex - 1u) + 0.5f) - g.cx));
-    const float Yb = fmaxf(fabsf(ylo), fabsf(yhi));
-    const float slack = kSlack * (g.a * X * X + 2.0f * fabsf(g.b) * X * Yb + g.c * Yb * Yb);
-    const float margin = 0x1p-20f * (fabsf(g.cx) + (float)W);
-    float xa = 0.0f, xb = 0.0f;
-    d.sure = band_extent(g.a, g.b, g.ia, g.ic, S.det, S.sa, S.sc, g.cutoff - slack, ylo, yhi, xa, xb)
-                 ? columns_meeting(xa, xb, g.cx, margin, T, W, tx0, c0, c1)
-                 : 0u;
-    uint32_t maybe = 0u;
-    if (band_extent(g.a, g.b, g.ia, g.ic, S.det, S.sa, S.sc, g.cutoff + slack, ylo, yhi, xa, xb)) {
-        // (An extent that is not one -- a NaN -- leaves every column to the test.)
-        maybe = xa <= xb ? columns_meeting(xa, xb, g.cx, -margin, T, W, tx0, c0, c1)
-                         : ((2u << (c1 - c0)) - 1u) << (c0 - tx0);
-    }
-    d.test = maybe & ~d.sure;
-    return d;
-}
-
 // One strip entry for every (row, strip) a drawn footprint's rectangle
 // covers, rank by rank in depth order, a footprint's entries row by row and
 // left to right: key = its global strip, value = the rank. The rank's
