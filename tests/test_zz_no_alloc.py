@@ -5,6 +5,7 @@ memory taken by the context or by PyTorch's allocator during the calls, and
 the size limit refused with INVALID_ARGUMENT."""
 from __future__ import annotations
 
+import gc
 import sys
 
 import pytest
@@ -32,6 +33,9 @@ def test_noalloc_scan_matches_the_allocating_scan():
             out = torch.full((n,), -1, dtype=torch.int32, device="cuda:0")
             total = torch.full((1,), -1, dtype=torch.int64, device="cuda:0")
             torch.cuda.synchronize()
+            # What earlier tests left in cycles (a caught error holds its test's
+            # frame) goes now, not between the two readings.
+            gc.collect()
             held = raster.scratch_bytes()
             torch_held = torch.cuda.memory_allocated()
             raster.exclusive_scan_noalloc(values, out, total)
