@@ -347,7 +347,7 @@ hipError_t launch_contribution(const DView* views_dev, const uint32_t* tile_base
                                const uint32_t* pair_slots, const float* records, uint32_t mode, uint32_t* out,
                                hipStream_t s);
 hipError_t launch_blend_backward(const DView* views_dev, const uint32_t* tile_bases, uint32_t nviews,
-                                 uint32_t total_tiles, uint32_t tile, uint32_t batch, const uint32_t* ranges,
+                                 uint32_t total_tiles, uint32_t tile, const uint32_t* ranges,
                                  const uint32_t* pair_slots, const float* records, float* grad2d, hipStream_t s);
 hipError_t launch_project_backward(const ProjectArgs& a, const DView* views_dev, uint32_t nviews,
                                    const uint32_t* touched, const float* records, const float* grad2d,

@@ -3,20 +3,26 @@
 //
 // Forward: shaders/athenea/splat/splat_blend.slang:236-578 (splatBlend,
 // blendPixel with composite, matte and trace off, contributionMode 0). One
-// workgroup per tile, one thread per pixel; the tile's pairs are staged in
-// LDS `batch` at a time (the reference stages 256, splat_blend.slang:300-311)
-// and every pixel walks them from there. A wavefront whose 64 pixels are all
+// workgroup a tile of 8 or 16 pixels and four a tile of 32 (a 16 x 16 quarter
+// each), one thread per pixel; the tile's Gaussians are staged in LDS a batch
+// at a time (the reference stages 256, splat_blend.slang:300-311) and every
+// pixel walks the ones that meet its own 4 x 4 block, from that block's list.
+// A frame that keeps its walk for the adjoint stages listed pairs, `batch` at a
+// time (blend_kernel); a plain one picks the tile's Gaussians out of its strip
+// entries, in batches of its own (blend_entries_kernel); the variants and the
+// contributions walk listed pairs that meet 8 x 8 pixels (blend_ex_kernel,
+// contribution_kernel). A wavefront whose 64 pixels are all
 // done stops walking at once; the group stops loading when every wavefront
 // has stopped. Each pixel also keeps its final transmittance and how many of
 // its tile's pairs it read, which is all the adjoint needs to replay the walk.
 //
 // Adjoint: no counterpart in the reference. It walks the same pairs back to
-// front, recovering the transmittance before each Gaussian from the one
-// after it (T_k = T_{k+1} / (1 - alpha_k); alpha <= 0.99 keeps it stable),
-// and accumulates per-slot gradients of the centre, conic, alpha and colour.
-// The 16 lanes of a row walk the same pair at the same step, so a pair's
-// gradient is summed across the row first, then over the tile's rows in LDS,
-// and added to memory once a tile.
+// front from the same block lists, recovering the transmittance before each
+// Gaussian from the one after it (T_k = T_{k+1} / (1 - alpha_k); alpha <= 0.99
+// keeps it stable), and accumulates per-slot gradients of the centre, conic,
+// alpha and colour. The 16 lanes of a row walk one block's list, so a Gaussian's
+// gradient is summed across the row first, then over the tile's blocks in LDS,
+// and added to memory once a batch.
 #include "athx_internal.h"
 #include "bounds.h"
 
@@ -54,7 +60,7 @@ __device__ inline void stage(LdsBatch& s, uint32_t k, const float* records, uint
     s.colour[k] = make_float4(col.x, col.y, col.z, conic.y);
 }
 
-// A pair's record words as stage() reads them, and their LDS form.
+// A pair's record words.
 struct Staged {
     float4 screen, conic, col;
 };
@@ -62,12 +68,6 @@ struct Staged {
 __device__ inline Staged fetch(const float* records, uint32_t slot) {
     const float4* rec = reinterpret_cast<const float4*>(records + (size_t)slot * kRecordFloats);
     return Staged{rec[0], rec[1], rec[2]};
-}
-
-__device__ inline void put(LdsBatch& s, uint32_t k, const Staged& r) {
-    s.xy_cut_op[k] = make_float4(r.screen.x, r.screen.y, r.screen.w, r.conic.w);
-    s.conic[k] = make_float4(r.conic.x, 2.0f * r.conic.y, r.conic.z, r.screen.z);
-    s.colour[k] = make_float4(r.col.x, r.col.y, r.col.z, r.conic.y);
 }
 
 // e^(-power / 2) for a drawn pair: power <= the cut power <= 9, and above
@@ -1470,13 +1470,10 @@ hipError_t launch_contribution(const DView* views_dev, const uint32_t* tile_base
 }
 
 hipError_t launch_blend_backward(const DView* views_dev, const uint32_t* tile_bases, uint32_t nviews,
-                                 uint32_t total_tiles, uint32_t tile, uint32_t batch, const uint32_t* ranges,
+                                 uint32_t total_tiles, uint32_t tile, const uint32_t* ranges,
                                  const uint32_t* pair_slots, const float* records, float* grad2d, hipStream_t s) {
     if (total_tiles == 0) {
         return hipSuccess;
-    }
-    if (batch == 0 || batch > kMaxBatch) {
-        return hipErrorInvalidValue;
     }
     switch (tile) {
     case 8:

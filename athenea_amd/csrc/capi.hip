@@ -1157,9 +1157,8 @@ athx_status enqueue_backward(athx_ctx* ctx, const ProjectArgs& pa, uint32_t nvie
                              const athx_settings* settings, const athx_grads& grads, hipStream_t s) {
     ATHX_HIP(ctx, launch_fill_u32(as<uint32_t>(ctx->grad2d), 0u, (uint64_t)slots * kGrad2d, s), "clear gradients");
     ATHX_HIP(ctx, launch_blend_backward(as<DView>(ctx->views), as<uint32_t>(ctx->tile_bases), nviews, ctx->last_tiles,
-                                        settings->tile, settings->batch, as<uint32_t>(ctx->ranges),
-                                        as<uint32_t>(ctx->pair_vals), as<float>(ctx->records),
-                                        as<float>(ctx->grad2d), s),
+                                        settings->tile, as<uint32_t>(ctx->ranges), as<uint32_t>(ctx->pair_vals),
+                                        as<float>(ctx->records), as<float>(ctx->grad2d), s),
              "blend backward");
     ATHX_HIP(ctx, launch_project_backward(pa, as<DView>(ctx->views), nviews, as<uint32_t>(ctx->touched),
                                           as<float>(ctx->records), as<float>(ctx->grad2d), grads, s),

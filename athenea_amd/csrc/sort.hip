@@ -1,10 +1,11 @@
 // sort.hip -- stable LSD radix sort of (uint32 or uint64 key, uint32 value)
 // pairs for gfx950, onesweep (Adinets & Merrill 2022): one kernel counts every digit
 // pass's histogram in a single read of the keys, then one kernel a pass
-// ranks each 4096-key partition in LDS with wavefront ballots (a 64-lane
-// match on the 8 digit bits), finds where its digits start among the
-// partitions before it by decoupled look-back, and writes each digit's run
-// out contiguously from LDS.
+// ranks each partition (1024 keys of a small sort, 4096 of a larger one) in LDS
+// with wavefront ballots (a 64-lane match on the 8 digit bits), finds where its
+// digits start among the partitions before it by decoupled look-back, and
+// writes each digit's run out contiguously from LDS. Sorts past kReduceScanMin
+// keys, and segmented ones, count, scan and scatter instead.
 //
 // Semantics: gpu::RadixSort::sort (modules/gpu/include/athenea/gpu/algo/
 // RadixSort.h:63-64; modules/gpu/src/algo/RadixSort.cpp:95-261), a stable

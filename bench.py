@@ -79,11 +79,12 @@ def stage_bytes(n: int, visible: int, entries: int, tiles: int, pixels: int, rel
         "depth_sort": n * 4 + visible * 8 + 3 * visible * 16,
         "counts": visible * 8,
         # the sorted slot and the record's 32 B of geometry read a drawn
-        # footprint; (strip | tile mask, slot) written an entry
-        "emit": visible * (4 + 32) + entries * 8,
-        # no pairs are listed: each strip's two bounds written
+        # footprint; (strip | tile mask, slot) written an entry; each strip's
+        # two bounds written
+        "emit": visible * (4 + 32) + entries * 8 + tiles // 16 * 8,
+        # no pairs are listed, and no tile's range
         "tile_sort": 0,
-        "ranges": tiles // 16 * 8,
+        "ranges": 0,
         # each entry's tile mask and slot and each drawn record read once,
         # colour and depth written
         "blend": entries * 8 + visible * 48 + pixels * 20,

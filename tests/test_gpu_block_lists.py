@@ -55,9 +55,9 @@ def gradients(raster, cloud, view, dl, settings):
 
 @pytest.mark.parametrize("size", [(101, 67), (3, 130)])
 def test_adjoint_over_several_batches(raster, size):
-    """Tiles of hundreds of pairs, many batches of every tile side's adjoint
-    (32, 56 and 24 Gaussians): the gradients of one picture do not depend on
-    how its pairs are cut up. Each is a sum of at most a few thousand float
+    """Tiles of hundreds of pairs, many batches of every tile side's adjoint (32
+    Gaussians of a tile of 8, 56 of the others): the gradients of one picture do
+    not depend on how its pairs are cut up. Each is a sum of at most a few thousand float
     products in another order, so they agree to a few thousand units of 2^-24
     of the largest."""
     print("adjoint batches", size, flush=True)
