@@ -70,10 +70,15 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t x, uint32_t* s_tmp, uin
 // kSmallSort, 4096 beyond. A few thousand to a few hundred thousand keys are
 // few partitions of 4096, each a CU's whole latency chain (ranking 16 keys a
 // lane one after another) on a tenth of the chip: four times the partitions
-// take a quarter of the chain. Measured, us a pass of 4 k and 100 k keys:
-// 11.0 and 14.2 with 4096 and one predecessor a look-back step, 5.9 and 9.9
-// with 1024 and kLook; 1.3 M keys take 24.4 and (4096, kLook) 22.8.
-constexpr uint32_t kSmallSort = 1u << 19;
+// take a quarter of the chain, and look back four times as far. Measured, us a
+// sort with partitions of 1024 and of 4096 keys:
+//   keys      32-bit, 24 bits sorted    64-bit, 32 bits sorted
+//   4 096       29.4     45.4             38.4     56.2
+//   65 536      37.9     51.4             49.2     64.3
+//   262 144     50.9     56.5             67.6     72.1
+//   393 216     64.8     60.7             82.6     76.2
+//   524 288     73.2     62.8             96.7     81.6
+constexpr uint32_t kSmallSort = 1u << 18;
 __host__ __device__ inline uint32_t onesweep_part(uint32_t cap) {
     return cap <= kSmallSort ? kThreads * 4u : kThreads * kItems;
 }
