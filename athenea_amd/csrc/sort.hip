@@ -15,7 +15,7 @@
 #include "athx_internal.h"
 
 #ifndef ATHX_REDUCE_SCAN_MIN
-#define ATHX_REDUCE_SCAN_MIN (1u << 22)
+#define ATHX_REDUCE_SCAN_MIN (1u << 21)
 #endif
 
 namespace athx {
@@ -129,6 +129,15 @@ __device__ inline uint64_t match_digit(uint32_t d, uint32_t width, bool ok) {
 constexpr uint32_t kHistBlocks = 1024;
 // Sorts of at least this capacity take the reduce-scan-scatter passes;
 // smaller ones onesweep's, whose few partitions wait little on each other.
+// Measured, us a sort by onesweep (4096-key partitions, kLook predecessors a
+// look-back step) and by reduce-scan-scatter:
+//   keys         32-bit, 24 bits sorted    64-bit, 32 bits sorted
+//   524 288        62.8     71.7             81.6     98.6
+//   1 048 576      75.5     80.2            100.5    115.0
+//   2 097 152      97.7     88.3            130.6    121.7
+//   4 194 304     146.9    103.1            209.1    201.6
+//   10 000 000    247.7    200.3            402.3    376.4
+//   33 554 432    723.3    579.1          1 210     1 154
 constexpr uint32_t kReduceScanMin = ATHX_REDUCE_SCAN_MIN;
 
 template <typename K>
