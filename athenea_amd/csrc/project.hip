@@ -768,10 +768,51 @@ __global__ void __launch_bounds__(kSmallThreads) count_small_kernel(const DView*
 
 // Where each key's entries start and end among the sorted keys; a key with
 // none gets (0, 0), as splat_tiles_clear.slang:8-17 and splat_ranges.slang:
-// 11-25 leave a tile. A wavefront a key: its halves look for the first entry
-// of the key and of the one after it, 32 probes a step (12 M entries: five
-// steps of one memory latency, where a lane's binary search took 24: 15.6 us
-// a launch that way, 5.2 this).
+// 11-25 leave a tile. Up to kWaveRanges keys a wavefront takes one: its halves
+// look for the first entry of the key and of the one after it, 32 probes a step
+// (12 M entries: five steps of one memory latency, where a lane's binary search
+// takes 24). Past that the wavefronts no longer fit the chip at once, and a lane
+// a key is faster again. Measured, us a launch with a wavefront a key and with a
+// lane a key:
+//   keys        100 000 entries    12 M entries
+//   500           6.2     8.6        6.2    10.8
+//   8 192         6.4     7.8        7.4    10.4
+//   16 384        8.6     7.7       13.5    10.3
+//   65 536       19.8     7.8       30.0    14.9
+//   1 048 576   230      17.4      356      41.8
+constexpr uint32_t kWaveRanges = 8192;
+
+__device__ inline uint32_t lower_bound_key(const uint32_t* keys, uint32_t n, uint64_t key, uint32_t key_mask) {
+    uint32_t lo = 0, hi = n;
+    while (lo < hi) {
+        const uint32_t mid = lo + ((hi - lo) >> 1);
+        if ((uint64_t)(keys[mid] & key_mask) < key) {
+            lo = mid + 1;
+        } else {
+            hi = mid;
+        }
+    }
+    return lo;
+}
+
+__global__ void __launch_bounds__(256) ranges_lane_kernel(const uint32_t* __restrict__ keys,
+                                                          const uint64_t* __restrict__ n_dev, uint32_t cap,
+                                                          uint32_t tiles, uint32_t key_mask,
+                                                          uint32_t* __restrict__ ranges,
+                                                          const uint64_t* __restrict__ tally,
+                                                          uint64_t* __restrict__ pair_total) {
+    sum_tally(tally, pair_total);
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= tiles) {
+        return;
+    }
+    const uint32_t n = *n_dev < cap ? (uint32_t)*n_dev : cap;
+    const uint32_t start = lower_bound_key(keys, n, t, key_mask);
+    const uint32_t end = lower_bound_key(keys, n, (uint64_t)t + 1, key_mask);
+    ranges[2 * t] = start < end ? start : 0u;
+    ranges[2 * t + 1] = start < end ? end : 0u;
+}
+
 __global__ void __launch_bounds__(256) ranges_kernel(const uint32_t* __restrict__ keys,
                                                      const uint64_t* __restrict__ n_dev, uint32_t cap, uint32_t tiles,
                                                      uint32_t key_mask,
@@ -1713,8 +1754,9 @@ hipError_t launch_ranges(const uint32_t* sorted_keys, const uint64_t* n_dev, uin
     if (tiles == 0) {
         return hipSuccess;
     }
-    hipLaunchKernelGGL(ranges_kernel, dim3(div_up(tiles, 4)), dim3(256), 0, s, sorted_keys, n_dev, cap, tiles,
-                       key_mask, ranges, tally, pair_total);
+    const bool lanes = tiles > kWaveRanges;
+    hipLaunchKernelGGL(lanes ? ranges_lane_kernel : ranges_kernel, dim3(div_up(tiles, lanes ? 256u : 4u)), dim3(256), 0,
+                       s, sorted_keys, n_dev, cap, tiles, key_mask, ranges, tally, pair_total);
     return hipGetLastError();
 }
 

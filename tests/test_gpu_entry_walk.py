@@ -65,6 +65,17 @@ def test_several_views(raster, sizes):
     both(raster, cloud, views + [camera.view_for(away, 64, 48)], RenderSettings())
 
 
+@pytest.mark.parametrize("size,strips", [((257, 65535), 8192), ((513, 43690), 8193)])
+def test_about_the_strip_ranges_routes(raster, size, strips):
+    """The most strips whose ranges a wavefront each finds, and one more."""
+    print("entry walk strips", size, flush=True)
+    cloud = GaussianCloud.from_numpy(synthetic.make_cloud(3000, 5, log_scale_mean=-4.0, axis_spread=0.7), "cuda:0")
+    _, stats = both(raster, cloud, [a_view(*size, radius=0.1)], RenderSettings())
+    assert raster.frame_info()["strips"] == strips and stats.pairs > 1000
+    ranges = raster.frame_buffers()["ranges"].long()
+    assert int((ranges[:, 1] - ranges[:, 0]).sum()) == stats.pairs
+
+
 def test_readers_after_a_frame_without_pairs(raster):
     print("entry walk readers", flush=True)
     cloud = GaussianCloud.from_numpy(synthetic.make_cloud(5000, 7), "cuda:0")
