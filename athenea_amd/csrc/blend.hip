@@ -184,8 +184,8 @@ __device__ inline uint64_t band_mask(const LdsBatch& s, const Band& B, uint32_t 
 // 1600 x 1100: 403 us a launch, against 8 x 8 pixels a step's 278).
 //
 // Measured against walking what meets a wavefront's 8 x 8 pixels, one Gaussian
-// a step (us a launch, MI355X): 100 k Gaussians at 512 x 512 109 -> 57, 1.4 M
-// at 1920 x 1080 244 -> 201, the 60-view walk 3 340 -> 2 420, 20 M in eight
+// a step (us a launch, MI355X): 100 k Gaussians at 512 x 512 109 -> 61, 1.4 M
+// at 1920 x 1080 244 -> 206, the 60-view walk 3 340 -> 2 420, 20 M in eight
 // views 3 415 -> 2 045.
 constexpr uint32_t kBlock = 4;  // a block's side, pixels
 
@@ -508,7 +508,7 @@ __global__ void __launch_bounds__(TILE * TILE) blend_kernel(const DView* __restr
 // hit one entry in sixteen, and a batch costs its barriers and its block tests
 // whatever it holds.
 // Measured against listing the pairs and blend_kernel over them (us a frame's
-// GPU time, MI355X): 4 k Gaussians at 203 x 117 137 -> 114, 100 k at 512 x 512
+// GPU time, the other passes as they then were, MI355X): 4 k Gaussians at 203 x 117 137 -> 114, 100 k at 512 x 512
 // 223 -> 190, 1.4 M at 1920 x 1080 924 -> 813, the 60-view walk 15 900 ->
 // 14 634, 20 M in eight views 18 000 -> 16 550, 0.9 M at 294 x 262 (many
 // entries a strip, most behind an opaque front) 583 -> 427.
@@ -1124,9 +1124,11 @@ __device__ inline void row_sum9(const float (&v)[9], float& x0, float& x1, float
 // the adds the walk was bound by that pipe at 95 %): the batch is what leaves
 // room for four workgroups a CU. Measured against the
 // walk of 8 x 8 pixels a step with whole-wavefront sums (us a launch, MI355X):
-// 100 k Gaussians at 512 x 512 293 -> 140, 1.4 M at 1920 x 1080 665 -> 461.
-// Tiles in dispatch order: banded over the XCDs the first takes 183 (the
-// middle bands hold most of the work), the second the same 461.
+// 100 k Gaussians at 512 x 512 293 -> 150, 1.4 M at 1920 x 1080 702 -> 501.
+// Bound by the VALU's issue (0.51 of its rate) with the LDS pipe serving
+// accesses in 0.28 of the clocks. Tiles in dispatch order: banded over the XCDs
+// the first took 183 where it took 140 (the middle bands hold most of the work),
+// the second the same.
 template <uint32_t TILE>
 constexpr uint32_t back_batch() {
     return TILE == 8 ? 32u : 56u;
