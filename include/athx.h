@@ -307,7 +307,8 @@ typedef struct athx_targets {
  * strip entries scanned in depth order; their emission, sorted on the strip
  * (project_ms .. emit_ms); the binning of the entries into tile-sorted pairs
  * in place of the reference's sort of the pair keys (tile_sort_ms); tile
- * ranges; blend. */
+ * ranges; blend. A frame that lists no pairs (athx_render_async) spends no time
+ * on binning and tile ranges: its strips' ranges are in emit_ms. */
 typedef struct athx_frame_stats {
     uint32_t splats;
     uint32_t visible;
